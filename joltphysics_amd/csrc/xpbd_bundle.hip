@@ -1,16 +1,15 @@
 // Bundle kernel: several LDS-resident soft bodies per workgroup.
 //
-// One 256-thread workgroup owns a bundle of bodies for a whole xpbd_update call
-// (all frames x collision steps x iterations).  All positions + inverse masses
-// of the bundle live in LDS as float4.  Each body's constraint program -- the
+// One workgroup of 512 or 1024 threads owns a bundle of bodies for a whole
+// xpbd_update call (all frames x collision steps x iterations).  All positions +
+// inverse masses of the bundle live in LDS.  Each body's constraint program -- the
 // merged levels of its parallel update groups followed by the levels of its
 // non-parallel group (SoftBodyMotionProperties.cpp:1030-1115) -- is merged with
 // the other bodies' programs by level index, so the lanes of a level are filled
 // by constraints of several bodies.  Bodies are independent (they share no
 // vertices), so merging keeps every body's own sequential order and the results
-// stay bit-identical to the reference.  Within a level the host groups records
-// by constraint type and pads the groups to whole wavefronts, so a wavefront
-// runs one constraint path instead of the union of all of them.
+// stay bit-identical to the reference.  The merged levels run as a task program:
+// within a level the host hands each wavefront records of one constraint type.
 //
 // Per-vertex phases look up their body through a per-vertex body slot in LDS
 // and use that body's per-step constants (gravity, sub-step, damping, ...).
@@ -52,17 +51,15 @@ struct BodyLocal
 
 struct BundleLds
 {
-    uint32_t recs, lvl, vb, locals, states, total;
+    uint32_t vb, locals, states, total;
 };
 
 // pos_bytes: 16 (float4 position + inverse mass) or 12 (float3; one inverse mass per bundle)
-__host__ __device__ inline BundleLds bundle_layout(uint32_t nv, uint32_t nrec, uint32_t nlvl, uint32_t nb, uint32_t pos_bytes)
+__host__ __device__ inline BundleLds bundle_layout(uint32_t nv, uint32_t nb, uint32_t pos_bytes)
 {
     BundleLds l;
     uint32_t off = (nv * pos_bytes + 15u) & ~15u;
-    l.recs = off; off += nrec * 16u;
-    l.lvl = off; off += nlvl * 4u;
-    off = (off + 15u) & ~15u; l.vb = off; off += nv;
+    l.vb = off; off += nv;
     off = (off + 15u) & ~15u; l.locals = off; off += nb * (uint32_t)sizeof(BodyLocal);
     off = (off + 15u) & ~15u; l.states = off; off += nb * (uint32_t)sizeof(BodyStateDev);
     l.total = (off + 15u) & ~15u;
@@ -89,7 +86,7 @@ template <> struct BundlePositions<true>
     }
 };
 
-template <bool STAGED, int BLOCK, bool UNIFORM, bool EXT>
+template <int BLOCK, bool UNIFORM, bool EXT>
 __device__ __forceinline__ void bundle_update(
     const BundleDev &G, const BodyDev *__restrict__ bodies, BodyStateDev *__restrict__ states,
     const ColliderDev *__restrict__ colliders, uint32_t num_colliders,
@@ -102,12 +99,9 @@ __device__ __forceinline__ void bundle_update(
     const int wave = tid >> 6;
     const uint32_t nv = G.nv;
     const uint32_t nb = G.num_bodies;
-    const uint32_t nlev = G.nlev;
     const bool has_sleepers = G.has_sleepers != 0;
-    const BundleLds lay = bundle_layout(nv, STAGED ? G.num_records : 0u, STAGED ? G.nlev + 1 : 0u, nb, UNIFORM ? 12u : 16u);
+    const BundleLds lay = bundle_layout(nv, nb, UNIFORM ? 12u : 16u);
     const typename BundlePositions<UNIFORM>::Type X = BundlePositions<UNIFORM>::make(lds_raw, G.uniform_inv_mass);
-    const uint4 *recs = STAGED ? reinterpret_cast<const uint4 *>(lds_raw + lay.recs) : G.recs;
-    const uint32_t *lvl = STAGED ? reinterpret_cast<const uint32_t *>(lds_raw + lay.lvl) : G.lvl;
     uint8_t *vb = reinterpret_cast<uint8_t *>(lds_raw + lay.vb);
     BodyLocal *loc = reinterpret_cast<BodyLocal *>(lds_raw + lay.locals);
     BodyStateDev *st = reinterpret_cast<BodyStateDev *>(lds_raw + lay.states);
@@ -115,15 +109,6 @@ __device__ __forceinline__ void bundle_update(
     Leaf *leaves = reinterpret_cast<Leaf *>(G.leaves);
 
     // ---- launch prologue
-    if (STAGED)
-    {
-        uint4 *rd = reinterpret_cast<uint4 *>(lds_raw + lay.recs);
-        for (uint32_t i = tid; i < G.num_records; i += BLOCK)
-            rd[i] = G.recs[i];
-        uint32_t *ld = reinterpret_cast<uint32_t *>(lds_raw + lay.lvl);
-        for (uint32_t i = tid; i <= G.nlev; i += BLOCK)
-            ld[i] = G.lvl[i];
-    }
     for (uint32_t i = tid; i < nv; i += BLOCK)
         pset(X, i, G.x[i]);
     for (uint32_t b = 0; b < nb; ++b)
@@ -398,17 +383,12 @@ __device__ __forceinline__ void bundle_update(
 
                 // ---- merged level program of all bodies (skin records carry their entries)
                 const RecordCtx sk{ G.skin, 0u, (float)(it + 1) / (float)iterations };
+                TaskStream tasks;
+                tasks.begin(G.recs, G.desc, G.heads + wave, lane);
                 if (has_sleepers)
-                {
-                    auto skip = [&](const uint4 &r) { return r.x == kNopRecord || !st[vb[r.x & 0x3fffu]].active; };
-                    if (STAGED) run_levels_lds<BLOCK>(recs, lvl, nlev, X, inv_dt_sq, tid, skip, sk);
-                    else run_levels_global<BLOCK>(recs, lvl, nlev, X, inv_dt_sq, tid, skip, sk);
-                }
+                    tasks.run(X, inv_dt_sq, lane, [&](const uint4 &r) { return !st[vb[r.x & 0x3fffu]].active; }, sk);
                 else
-                {
-                    if (STAGED) run_levels_lds<BLOCK>(recs, lvl, nlev, X, inv_dt_sq, tid, NoSkip(), sk);
-                    else run_levels_global<BLOCK>(recs, lvl, nlev, X, inv_dt_sq, tid, NoSkip(), sk);
-                }
+                    tasks.run(X, inv_dt_sq, lane, NoSkip(), sk);
 
                 // ---- collision + velocity (SoftBodyMotionProperties.cpp:700-825), fused with the
                 // next integration (no pressure) or the per-vertex part of UpdateSoftBodyState.
@@ -653,62 +633,55 @@ __device__ __forceinline__ void bundle_update(
         *G.elapsed = __builtin_amdgcn_s_memrealtime() - t_begin;
 }
 
-// One workgroup per bundle.  STAGED: the records and level offsets are copied
-// into LDS at launch (small programs only, 256-thread launches); UNIFORM: three
-// floats per vertex in LDS and the one inverse mass of the bundle.
-template <bool STAGED, int BLOCK, bool UNIFORM, bool EXT>
-__global__ __launch_bounds__(BLOCK) void bundle_kernel(
+// One workgroup per bundle.  UNIFORM: three floats per vertex in LDS and the one
+// inverse mass of the bundle.
+// Four wavefronts per SIMD, so that two 512-thread workgroups share a CU: at most 128 registers.
+template <int BLOCK, bool UNIFORM, bool EXT>
+__global__ __launch_bounds__(BLOCK, 4) void bundle_kernel(
     const BundleDev *__restrict__ bundles, const BodyDev *__restrict__ bodies, BodyStateDev *__restrict__ states,
     const ColliderDev *__restrict__ colliders, uint32_t num_colliders,
     float gx, float gy, float gz, float dt, int32_t steps, int32_t frames)
 {
-    bundle_update<STAGED, BLOCK, UNIFORM, EXT>(bundles[blockIdx.x], bodies, states, colliders, num_colliders, gx, gy, gz, dt, steps, frames);
+    bundle_update<BLOCK, UNIFORM, EXT>(bundles[blockIdx.x], bodies, states, colliders, num_colliders, gx, gy, gz, dt, steps, frames);
 }
 
-uint32_t bundle_lds_bytes(uint32_t nv, uint32_t nrec, uint32_t nlvl, uint32_t nb, bool uniform)
+uint32_t bundle_lds_bytes(uint32_t nv, uint32_t nb, bool uniform)
 {
-    return bundle_layout(nv, nrec, nlvl, nb, uniform ? 12u : 16u).total;
+    return bundle_layout(nv, nb, uniform ? 12u : 16u).total;
 }
 
 uint32_t bundle_leaf_bytes() { return (uint32_t)sizeof(Leaf); }
 
-template <bool S, int BLOCK, bool U, bool EXT>
+template <int BLOCK, bool U, bool EXT>
 static hipError_t launch_bundles_variant(const BundleDev *bundles, uint32_t num_bundles, const BodyDev *bodies, BodyStateDev *states,
                                          const ColliderDev *colliders, uint32_t num_colliders, uint32_t lds_bytes,
                                          float gx, float gy, float gz, float dt, int32_t steps, int32_t frames, hipStream_t stream)
 {
-    static const hipError_t configured = hipFuncSetAttribute((const void *)bundle_kernel<S, BLOCK, U, EXT>,
+    static const hipError_t configured = hipFuncSetAttribute((const void *)bundle_kernel<BLOCK, U, EXT>,
                                                              hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024 - 1024);
     if (configured != hipSuccess)
         return configured;
-    hipLaunchKernelGGL((bundle_kernel<S, BLOCK, U, EXT>), dim3(num_bundles), dim3(BLOCK), lds_bytes, stream,
+    hipLaunchKernelGGL((bundle_kernel<BLOCK, U, EXT>), dim3(num_bundles), dim3(BLOCK), lds_bytes, stream,
                        bundles, bodies, states, colliders, num_colliders, gx, gy, gz, dt, steps, frames);
     return hipGetLastError();
 }
 
 template <bool U, bool EXT>
-static hipError_t launch_bundles_uniform(bool staged, uint32_t block, const BundleDev *bundles, uint32_t num_bundles,
+static hipError_t launch_bundles_uniform(uint32_t block, const BundleDev *bundles, uint32_t num_bundles,
                                          const BodyDev *bodies, BodyStateDev *states, const ColliderDev *colliders,
                                          uint32_t num_colliders, uint32_t lds_bytes, float gx, float gy, float gz, float dt,
                                          int32_t steps, int32_t frames, hipStream_t stream)
 {
-    if (staged && block == 256)
-        return launch_bundles_variant<true, 256, U, EXT>(bundles, num_bundles, bodies, states, colliders, num_colliders, lds_bytes, gx, gy, gz, dt, steps, frames, stream);
-    if (staged)
-        return hipErrorInvalidValue;
     if (block == 1024)
-        return launch_bundles_variant<false, 1024, U, EXT>(bundles, num_bundles, bodies, states, colliders, num_colliders, lds_bytes, gx, gy, gz, dt, steps, frames, stream);
+        return launch_bundles_variant<1024, U, EXT>(bundles, num_bundles, bodies, states, colliders, num_colliders, lds_bytes, gx, gy, gz, dt, steps, frames, stream);
     if (block == 512)
-        return launch_bundles_variant<false, 512, U, EXT>(bundles, num_bundles, bodies, states, colliders, num_colliders, lds_bytes, gx, gy, gz, dt, steps, frames, stream);
-    if (block == 256)
-        return launch_bundles_variant<false, 256, U, EXT>(bundles, num_bundles, bodies, states, colliders, num_colliders, lds_bytes, gx, gy, gz, dt, steps, frames, stream);
+        return launch_bundles_variant<512, U, EXT>(bundles, num_bundles, bodies, states, colliders, num_colliders, lds_bytes, gx, gy, gz, dt, steps, frames, stream);
     return hipErrorInvalidValue;
 }
 
-// block: 256, 512 or 1024 threads (staged bundles only in 256-thread launches); uniform:
-// the bundles' vertices share one inverse mass and keep three floats per vertex in LDS;
-// ext: the collider list holds triangle trees or scaled convex hulls
-hipError_t launch_bundles(bool staged, uint32_t block, bool uniform, bool ext, const BundleDev *bundles, uint32_t num_bundles,
+// block: 512 or 1024 threads; uniform: the bundles' vertices share one inverse mass and keep
+// three floats per vertex in LDS; ext: the collider list holds triangle trees or scaled convex hulls
+hipError_t launch_bundles(uint32_t block, bool uniform, bool ext, const BundleDev *bundles, uint32_t num_bundles,
                           const BodyDev *bodies, BodyStateDev *states, const ColliderDev *colliders, uint32_t num_colliders,
                           uint32_t lds_bytes, float gx, float gy, float gz, float dt, int32_t steps, int32_t frames,
                           hipStream_t stream)
@@ -716,14 +689,10 @@ hipError_t launch_bundles(bool staged, uint32_t block, bool uniform, bool ext, c
     if (num_bundles == 0)
         return hipSuccess;
     if (ext)
-    {
-        if (uniform)
-            return launch_bundles_uniform<true, true>(staged, block, bundles, num_bundles, bodies, states, colliders, num_colliders, lds_bytes, gx, gy, gz, dt, steps, frames, stream);
-        return launch_bundles_uniform<false, true>(staged, block, bundles, num_bundles, bodies, states, colliders, num_colliders, lds_bytes, gx, gy, gz, dt, steps, frames, stream);
-    }
-    if (uniform)
-        return launch_bundles_uniform<true, false>(staged, block, bundles, num_bundles, bodies, states, colliders, num_colliders, lds_bytes, gx, gy, gz, dt, steps, frames, stream);
-    return launch_bundles_uniform<false, false>(staged, block, bundles, num_bundles, bodies, states, colliders, num_colliders, lds_bytes, gx, gy, gz, dt, steps, frames, stream);
+        return uniform ? launch_bundles_uniform<true, true>(block, bundles, num_bundles, bodies, states, colliders, num_colliders, lds_bytes, gx, gy, gz, dt, steps, frames, stream)
+                       : launch_bundles_uniform<false, true>(block, bundles, num_bundles, bodies, states, colliders, num_colliders, lds_bytes, gx, gy, gz, dt, steps, frames, stream);
+    return uniform ? launch_bundles_uniform<true, false>(block, bundles, num_bundles, bodies, states, colliders, num_colliders, lds_bytes, gx, gy, gz, dt, steps, frames, stream)
+                   : launch_bundles_uniform<false, false>(block, bundles, num_bundles, bodies, states, colliders, num_colliders, lds_bytes, gx, gy, gz, dt, steps, frames, stream);
 }
 
 } // namespace xpbd

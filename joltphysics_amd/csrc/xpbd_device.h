@@ -252,6 +252,231 @@ __device__ __forceinline__ void project_lra(const P &X, uint32_t i0, uint32_t i1
         pset(X, i1, f4(x0 + (delta * max_distance) / sqrtf(delta_len_sq), p1.w));
 }
 
+// ---------------------------------------------------------------- divisions and square roots
+// Correctly rounded through the double unit, which issues a fused multiply-add at the float
+// rate on gfx950.  A quotient of two floats lies at least 2^-49 (relative) from every midpoint
+// of neighbouring floats, a square root at least 2^-51, so a double result closer than that
+// rounds to the correctly rounded float: one cubic step takes the 24-bit hardware seeds to
+// double's own rounding error (about 2^-52 for a quotient, 2^-52.4 for a root).
+//
+// sqrtf(x): 10 instructions where the compiler's form takes 18 (76 against 112 cycles as a
+// dependent chain of one wavefront).
+constexpr int kClassZeroOrInf = 0x020 | 0x040 | 0x200;                          // -0, +0, +inf
+__device__ __forceinline__ float square_root(float x)
+{
+    const double d = (double)x;
+    const double y = __builtin_amdgcn_rsq(d);
+    const double s = d * y;
+    const double e = __builtin_fma(-s, y, 1.0);
+    const float r = (float)__builtin_fma(s, e * __builtin_fma(e, 0.375, 0.5), s);
+    return __builtin_amdgcn_classf(x, kClassZeroOrInf) ? x : r;
+}
+// Three quotients of one denominator: 14 instructions where three plain divisions take 33.  A
+// quotient that this does not cover sets `redo` (denormal results, where an exact tie is
+// possible, infinities and NaN); the caller then takes the plain divisions.  A single quotient
+// gains nothing over the plain division.
+constexpr int kClassRedo = 0x001 | 0x002 | 0x004 | 0x200 | 0x010 | 0x080;       // NaN, infinite, denormal
+__device__ __forceinline__ V3 divide3(V3 a, float b, bool &redo)
+{
+    const double d = (double)b;
+    const double r0 = __builtin_amdgcn_rcp(d);
+    const double e = __builtin_fma(-d, r0, 1.0);
+    const double r = __builtin_fma(r0, __builtin_fma(e, e, e), r0);
+    const V3 q = v3((float)((double)a.x * r), (float)((double)a.y * r), (float)((double)a.z * r));
+    redo = redo || __builtin_amdgcn_classf(q.x, kClassRedo) || __builtin_amdgcn_classf(q.y, kClassRedo)
+           || __builtin_amdgcn_classf(q.z, kClassRedo);
+    return q;
+}
+// ACosApproximate (acos_approx) with this square root
+__device__ __forceinline__ float acos_approx_device(float x)
+{
+    const float ax = fabsf(x);
+    const float abs_x = ax < 1.0f ? ax : 1.0f;
+    const float val = square_root(1.0f - abs_x) * (kPi / 2 - 0.175394f * abs_x);
+    return x < 0.0f ? kPi - val : val;
+}
+
+// ---------------------------------------------------------------- wide levels: one lane per constraint
+// The projections of the level programs where a level fills the workgroup and the issue rate
+// bounds it: one lane per constraint, no exit before the stores, quotients that share a
+// denominator through divide3.  The first wavefront with a quotient divide3 does not cover
+// takes the plain projection instead (nothing is stored before that is known).
+template <class P>
+__device__ __forceinline__ void project_edge_wide(const P &X, uint32_t i0, uint32_t i1, float rest, float compliance, float inv_dt_sq)
+{
+    const float4 p0 = pget(X, i0), p1 = pget(X, i1);
+    const V3 x0 = xyz(p0), x1 = xyz(p1);
+    const float w0 = p0.w, w1 = p1.w;
+    const V3 delta = x1 - x0;
+    const float length = square_root(len_sq(delta));
+    const float denom = length * ((w0 + w1) + compliance * inv_dt_sq);
+    bool redo = false;
+    const V3 correction = divide3(delta * (length - rest), denom, redo);
+    const bool skip = denom < 1.0e-12f;
+    if (__builtin_expect(__builtin_amdgcn_ballot_w64(redo && !skip) != 0ull, 0))
+        project_edge(X, i0, i1, rest, compliance, inv_dt_sq);
+    else if (!skip)
+    {
+        pset(X, i0, f4(x0 + w0 * correction, w0));
+        pset(X, i1, f4(x1 - w1 * correction, w1));
+    }
+}
+
+template <class P>
+__device__ __forceinline__ void project_bend_wide(const P &X, uint32_t i0, uint32_t i1, uint32_t i2, uint32_t i3, float compliance,
+                                                  float initial_angle, float inv_dt_sq)
+{
+    const float4 p0 = pget(X, i0), p1 = pget(X, i1), p2 = pget(X, i2), p3 = pget(X, i3);
+    const V3 x0 = xyz(p0), x1 = xyz(p1), x2 = xyz(p2), x3 = xyz(p3);
+    const V3 e = x1 - x0;
+    const float e_len = square_root(len_sq(e));
+    const V3 x1x2 = x2 - x1;
+    const V3 x1x3 = x3 - x1;
+    V3 n1 = cross(x2 - x0, x1x2);
+    V3 n2 = cross(x1x3, x3 - x0);
+    const float n1_len_sq = len_sq(n1);
+    const float n2_len_sq = len_sq(n2);
+    const float n1n2 = n1_len_sq * n2_len_sq;
+    bool skip = e_len < 1.0e-6f || n1n2 < 1.0e-24f;
+    const float sign = sign_of(dot(cross(n2, n1), e));
+    const float d = dot(n1, n2) / square_root(n1n2);
+    float c = sign * acos_approx_device(d) - initial_angle;
+    const float c_down = c - 2.0f * kPi, c_up = c + 2.0f * kPi;
+    c = c > kPi ? c_down : c < -kPi ? c_up : c;
+    bool redo = false;
+    n1 = divide3(n1, n1_len_sq, redo);
+    n2 = divide3(n2, n2_len_sq, redo);
+    const V3 d0c = divide3(dot(x1x2, e) * n1 + dot(x1x3, e) * n2, e_len, redo);
+    const V3 d2c = e_len * n1;
+    const V3 d3c = e_len * n2;
+    const V3 d1c = (neg(d0c) - d2c) - d3c;
+    const float w0 = p0.w, w1 = p1.w, w2 = p2.w, w3 = p3.w;
+    const float denom = (((w0 * len_sq(d0c) + w1 * len_sq(d1c)) + w2 * len_sq(d2c)) + w3 * len_sq(d3c)) + compliance * inv_dt_sq;
+    const float minus_lambda = c / denom;
+    if (__builtin_expect(__builtin_amdgcn_ballot_w64(redo && !skip) != 0ull, 0))
+        project_bend(X, i0, i1, i2, i3, compliance, initial_angle, inv_dt_sq);
+    else if (!skip && !(denom < 1.0e-12f))
+    {
+        pset(X, i0, f4(x0 - (minus_lambda * w0) * d0c, w0));
+        pset(X, i1, f4(x1 - (minus_lambda * w1) * d1c, w1));
+        pset(X, i2, f4(x2 - (minus_lambda * w2) * d2c, w2));
+        pset(X, i3, f4(x3 - (minus_lambda * w3) * d3c, w3));
+    }
+}
+
+// ---------------------------------------------------------------- narrow levels: four lanes per constraint
+// The same projections on a quad of lanes: lanes 0, 1 and 2 hold the x, y and z components of
+// every vector, lane 3 repeats z.  A vector operation is one instruction instead of three, a
+// vector divided by a scalar one division; components move between the lanes as DPP operands.
+// Every component is computed with the reference's operations in its order.  What bounds a
+// narrow level is the instruction count of its longest constraint (a lone wavefront issues one
+// in 4 to 5 cycles): a bend takes about 200 where two lanes took 316 and one lane 354, a volume
+// 90 instead of 137, an edge 40 instead of 79.
+template <int CTRL>
+__device__ __forceinline__ float quad_perm(float v)
+{
+    return __int_as_float(__builtin_amdgcn_mov_dpp(__float_as_int(v), CTRL, 0xf, 0xf, true));
+}
+constexpr int kQuadX = 0x00, kQuadY = 0x55, kQuadZ = 0xaa;      // component to every lane
+constexpr int kQuadYZX = 0x09;                                  // [1, 2, 0, 0]
+// dot = (x x' + y y') + z z', in every lane
+__device__ __forceinline__ float quad_sum(float p) { return (quad_perm<kQuadX>(p) + quad_perm<kQuadY>(p)) + quad_perm<kQuadZ>(p); }
+__device__ __forceinline__ float quad_dot(float a, float b) { return quad_sum(a * b); }
+// cross product: (a b.yzx - a.yzx b).yzx
+__device__ __forceinline__ float quad_cross(float a, float b)
+{
+    return quad_perm<kQuadYZX>(a * quad_perm<kQuadYZX>(b) - quad_perm<kQuadYZX>(a) * b);
+}
+
+// Component `c` of vertex i, its inverse mass, and its store (lane 3 stores z again)
+__device__ __forceinline__ float cget(float4 *X, uint32_t i, uint32_t c) { return reinterpret_cast<const float *>(X)[4u * i + c]; }
+__device__ __forceinline__ float wget(float4 *X, uint32_t i) { return X[i].w; }
+__device__ __forceinline__ void cset(float4 *X, uint32_t i, uint32_t c, float v) { reinterpret_cast<float *>(X)[4u * i + c] = v; }
+__device__ __forceinline__ float cget(const PositionsF3 &X, uint32_t i, uint32_t c) { return X.x[3u * i + c]; }
+__device__ __forceinline__ float wget(const PositionsF3 &X, uint32_t) { return X.w; }
+__device__ __forceinline__ void cset(const PositionsF3 &X, uint32_t i, uint32_t c, float v) { X.x[3u * i + c] = v; }
+
+template <class P>
+__device__ __forceinline__ void project_edge_quad(const P &X, uint32_t c, uint32_t i0, uint32_t i1, float rest, float compliance,
+                                                  float inv_dt_sq)
+{
+    const float x0 = cget(X, i0, c), x1 = cget(X, i1, c);
+    const float w0 = wget(X, i0), w1 = wget(X, i1);
+    const float delta = x1 - x0;
+    const float length = square_root(quad_dot(delta, delta));
+    const float denom = length * ((w0 + w1) + compliance * inv_dt_sq);
+    const float correction = (delta * (length - rest)) / denom;
+    if (!(denom < 1.0e-12f))
+    {
+        cset(X, i0, c, x0 + w0 * correction);
+        cset(X, i1, c, x1 - w1 * correction);
+    }
+}
+
+template <class P>
+__device__ __forceinline__ void project_bend_quad(const P &X, uint32_t k, uint32_t i0, uint32_t i1, uint32_t i2, uint32_t i3,
+                                                  float compliance, float initial_angle, float inv_dt_sq)
+{
+    const float x0 = cget(X, i0, k), x1 = cget(X, i1, k), x2 = cget(X, i2, k), x3 = cget(X, i3, k);
+    const float w0 = wget(X, i0), w1 = wget(X, i1), w2 = wget(X, i2), w3 = wget(X, i3);
+    const float e = x1 - x0;
+    const float x1x2 = x2 - x1;
+    const float x1x3 = x3 - x1;
+    float n1 = quad_cross(x2 - x0, x1x2);
+    float n2 = quad_cross(x1x3, x3 - x0);
+    const float e_len = square_root(quad_dot(e, e));
+    const float n1_len_sq = quad_dot(n1, n1);
+    const float n2_len_sq = quad_dot(n2, n2);
+    const float n1n2 = n1_len_sq * n2_len_sq;
+    const float sign = sign_of(quad_dot(quad_cross(n2, n1), e));
+    const float d = quad_dot(n1, n2) / square_root(n1n2);
+    float c = sign * acos_approx_device(d) - initial_angle;
+    const float c_down = c - 2.0f * kPi, c_up = c + 2.0f * kPi;
+    c = c > kPi ? c_down : c < -kPi ? c_up : c;
+    n1 = n1 / n1_len_sq;
+    n2 = n2 / n2_len_sq;
+    const float d0c = (quad_dot(x1x2, e) * n1 + quad_dot(x1x3, e) * n2) / e_len;
+    const float d2c = e_len * n1;
+    const float d3c = e_len * n2;
+    const float d1c = ((0.0f - d0c) - d2c) - d3c;
+    const float denom = (((w0 * quad_dot(d0c, d0c) + w1 * quad_dot(d1c, d1c)) + w2 * quad_dot(d2c, d2c)) + w3 * quad_dot(d3c, d3c))
+                        + compliance * inv_dt_sq;
+    const float minus_lambda = c / denom;
+    if (!(e_len < 1.0e-6f) && !(n1n2 < 1.0e-24f) && !(denom < 1.0e-12f))
+    {
+        cset(X, i0, k, x0 - (minus_lambda * w0) * d0c);
+        cset(X, i1, k, x1 - (minus_lambda * w1) * d1c);
+        cset(X, i2, k, x2 - (minus_lambda * w2) * d2c);
+        cset(X, i3, k, x3 - (minus_lambda * w3) * d3c);
+    }
+}
+
+template <class P>
+__device__ __forceinline__ void project_volume_quad(const P &X, uint32_t k, uint32_t i1, uint32_t i2, uint32_t i3, uint32_t i4,
+                                                    float six_rest_volume, float compliance, float inv_dt_sq)
+{
+    const float x1 = cget(X, i1, k), x2 = cget(X, i2, k), x3 = cget(X, i3, k), x4 = cget(X, i4, k);
+    const float w1 = wget(X, i1), w2 = wget(X, i2), w3 = wget(X, i3), w4 = wget(X, i4);
+    const float x1x2 = x2 - x1;
+    const float x1x3 = x3 - x1;
+    const float x1x4 = x4 - x1;
+    const float d4c = quad_cross(x1x2, x1x3);
+    const float c = fabsf(quad_dot(d4c, x1x4)) - six_rest_volume;
+    const float d1c = quad_cross(x4 - x2, x3 - x2);
+    const float d2c = quad_cross(x1x3, x1x4);
+    const float d3c = quad_cross(x1x4, x1x2);
+    const float denom = (((w1 * quad_dot(d1c, d1c) + w2 * quad_dot(d2c, d2c)) + w3 * quad_dot(d3c, d3c)) + w4 * quad_dot(d4c, d4c))
+                        + compliance * inv_dt_sq;
+    const float minus_lambda = c / denom;
+    if (!(denom < 1.0e-12f))
+    {
+        cset(X, i1, k, x1 - (minus_lambda * w1) * d1c);
+        cset(X, i2, k, x2 - (minus_lambda * w2) * d2c);
+        cset(X, i3, k, x3 - (minus_lambda * w3) * d3c);
+        cset(X, i4, k, x4 - (minus_lambda * w4) * d4c);
+    }
+}
+
 // ApplySkinConstraints body for one skinned vertex (SoftBodyMotionProperties.cpp:509-571).
 // The vertex's skin state is entry g of `skin`, four float4: previous and current
 // skinned position, normal, and {max distance multiplier, back stop radius, skin
@@ -533,6 +758,132 @@ __device__ __forceinline__ void run_levels_global(const uint4 *recs, const uint3
             project_record<RODS>(X, q, inv_dt_sq, sk);
     }, gsync);
 }
+
+// ---------------------------------------------------------------- task programs
+// A task program is a level program cut per wavefront.  A task is up to 64 lanes of one kind of
+// projection inside one level: records of one constraint type, one lane or four lanes each.
+// Every wavefront has its own list of tasks, its records contiguous in memory in task order, and
+// one descriptor word per task:
+//   bits 0-6   records (1-64; 1-16 for a four-lane kind)
+//   bits 7-9   kind (TaskKind)
+//   bits 10-31 workgroup barriers to pass before the task: one per level boundary since the
+//              wavefront's previous task that needs one
+// The host chooses kinds and wavefronts per level and leaves out the barrier between two levels
+// that the same single wavefront runs.  Descriptors are loaded six tasks ahead, records three
+// (ring of three registers, the loop unrolled three times so the ring never moves), all as vector
+// loads in program order, so a step waits for no load issued in the last two steps; the level
+// offsets of run_program_global are scalar loads whose latency, like its exec-masked kinds, is
+// paid in every level.  An empty level costs 80 ns here and 145 to 229 ns there; a level of a
+// 90 x 90 cloth (31 bends, 37 edges) 745 ns against 1,010, one of a 16-cell cube 485 against 590,
+// one of the coloured cloth (512 bends, 600 edges) 2,200 against 3,500 (512 threads).
+enum TaskKind : uint32_t { kTaskVolume = 0, kTaskBend = 1, kTaskEdge = 2, kTaskLRA = 3, kTaskVolumeQuad = 4, kTaskBendQuad = 5, kTaskEdgeQuad = 6 };
+constexpr uint32_t kTaskQuadBit = 4u << 7;
+
+struct TaskStream
+{
+    const uint4 *recs;          // next record to fetch
+    const uint32_t *desc;
+    uint32_t desc_offset;       // byte offset of the next descriptor (the same in every lane)
+    uint32_t count, trail;
+    uint32_t d0, d1, d2;        // descriptors of the fetched records (uniform)
+    uint32_t q0, q1, q2;        // the next three descriptors
+    RecordVec r0, r1, r2;
+
+    __device__ __forceinline__ uint32_t next_desc()
+    {
+        const uint32_t v = *(const __attribute__((address_space(1))) uint32_t *)(const void *)((const char *)desc + desc_offset);
+        desc_offset += 4u;
+        return v;
+    }
+    // the record of this lane, or the one behind the task's last
+    __device__ __forceinline__ RecordVec fetch(uint32_t d, uint32_t lane)
+    {
+        const uint32_t n = d & 127u;
+        const uint32_t i = (d & kTaskQuadBit) ? lane >> 2 : lane;
+        const RecordVec r = load_record(recs, i < n ? i : n);
+        recs += n;
+        return r;
+    }
+    // `head`: {first descriptor, tasks, first record, barriers after the last task} of this wavefront.
+    // Issues the first loads; the caller may do other work before run().
+    __device__ __forceinline__ void begin(const uint4 *all_recs, const uint32_t *all_desc, const uint4 *head, uint32_t lane)
+    {
+        // global stores of an earlier phase still pending would make every later wait a full one
+        __builtin_amdgcn_s_waitcnt(kWaitVmcntZero);
+        head = uniform_ptr(head);
+        const uint32_t first = load_level_offset(reinterpret_cast<const uint32_t *>(head), 0);
+        count = load_level_offset(reinterpret_cast<const uint32_t *>(head), 1);
+        recs = uniform_ptr(all_recs) + load_level_offset(reinterpret_cast<const uint32_t *>(head), 2);
+        trail = load_level_offset(reinterpret_cast<const uint32_t *>(head), 3);
+        desc = uniform_ptr(all_desc) + first;
+        desc_offset = 0u;
+        asm volatile("" : "+v"(desc_offset));       // a vector register: the loads stay vector loads
+        const uint32_t f0 = next_desc(), f1 = next_desc(), f2 = next_desc();
+        q0 = next_desc();
+        q1 = next_desc();
+        q2 = next_desc();
+        d0 = uniform(f0);
+        d1 = uniform(f1);
+        d2 = uniform(f2);
+        r0 = fetch(d0, lane);
+        asm volatile("" ::: "memory");
+        r1 = fetch(d1, lane);
+        asm volatile("" ::: "memory");
+        r2 = fetch(d2, lane);
+    }
+    template <class P, class Skip>
+    __device__ __forceinline__ void step(uint32_t &d, RecordVec &r, uint32_t &q, const P &X, float inv_dt_sq, uint32_t lane, Skip skip,
+                                         const RecordCtx &sk)
+    {
+        for (uint32_t k = d >> 10; k > 0; --k)
+            __syncthreads();
+        pin_record(r);
+        const uint32_t n = d & 127u, kind = (d >> 7) & 7u;
+        const uint32_t i0 = r.x & 0x3fffu, i1 = r.x >> 16, i2 = r.y & 0x3fffu, i3 = r.y >> 16;
+        const float p0 = __uint_as_float(r.z), p1 = __uint_as_float(r.w);
+        if (d & kTaskQuadBit)
+        {
+            if ((lane >> 2) < n && !skip(as_uint4(r)))
+            {
+                const uint32_t c = (lane & 3u) < 2u ? (lane & 3u) : 2u;
+                if (kind == kTaskBendQuad)
+                    project_bend_quad(X, c, i0, i1, i2, i3, p0, p1, inv_dt_sq);
+                else if (kind == kTaskEdgeQuad)
+                    project_edge_quad(X, c, i0, i1, p0, p1, inv_dt_sq);
+                else
+                    project_volume_quad(X, c, i0, i1, i2, i3, p0, p1, inv_dt_sq);
+            }
+        }
+        else if (lane < n && !skip(as_uint4(r)))
+        {
+            if (kind == kTaskEdge)
+                project_edge_wide(X, i0, i1, p0, p1, inv_dt_sq);
+            else if (kind == kTaskBend)
+                project_bend_wide(X, i0, i1, i2, i3, p0, p1, inv_dt_sq);
+            else if (kind == kTaskVolume)
+                project_volume(X, i0, i1, i2, i3, p0, p1, inv_dt_sq);
+            else if (i0 == i1)
+                project_skin(X, i0, r.y + sk.base, p0, p1, sk);
+            else
+                project_lra(X, i0, i1, p0);
+        }
+        d = uniform(q);
+        q = next_desc();
+        r = fetch(d, lane);
+    }
+    template <class P, class Skip>
+    __device__ __forceinline__ void run(const P &X, float inv_dt_sq, uint32_t lane, Skip skip, const RecordCtx &sk)
+    {
+        for (uint32_t t = 0; t < count; t += 3)
+        {
+            step(d0, r0, q0, X, inv_dt_sq, lane, skip, sk);
+            step(d1, r1, q1, X, inv_dt_sq, lane, skip, sk);
+            step(d2, r2, q2, X, inv_dt_sq, lane, skip, sk);
+        }
+        for (uint32_t k = trail; k > 0; --k)
+            __syncthreads();
+    }
+};
 
 // Level program with records and offsets in LDS: the first record of the next
 // level is read before the barrier (the barrier's LDS wait covers it).

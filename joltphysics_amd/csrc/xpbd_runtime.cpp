@@ -19,9 +19,9 @@
 
 namespace xpbd {
 uint32_t kernel_lds_bytes(bool resident, bool staged, const SettingsDev &s, uint32_t max_leaves, uint32_t nc, uint32_t nf);
-uint32_t bundle_lds_bytes(uint32_t nv, uint32_t nrec, uint32_t nlvl, uint32_t nb, bool uniform);
+uint32_t bundle_lds_bytes(uint32_t nv, uint32_t nb, bool uniform);
 uint32_t bundle_leaf_bytes();
-hipError_t launch_bundles(bool staged, uint32_t block, bool uniform, bool ext, const BundleDev *bundles, uint32_t num_bundles,
+hipError_t launch_bundles(uint32_t block, bool uniform, bool ext, const BundleDev *bundles, uint32_t num_bundles,
                           const BodyDev *bodies, BodyStateDev *states, const ColliderDev *colliders, uint32_t num_colliders,
                           uint32_t lds_bytes, float gx, float gy, float gz, float dt, int32_t steps, int32_t frames,
                           hipStream_t stream);
@@ -128,6 +128,8 @@ struct xpbd_settings
     DevBuf<uint4> recs;
     DevBuf<uint32_t> lvl;
     DevBuf<WindowDev> windows;
+    DevBuf<uint4> task_recs, task_heads;    // task programs of the gathered windows
+    DevBuf<uint32_t> task_desc;
     DevBuf<uint32_t> vlist;
     DevBuf<uint32_t> faces, vf_begin, vf_list;
     SettingsDev dev{};
@@ -154,6 +156,7 @@ struct xpbd_settings
     // streamed bodies: the parallel-group windows (host copy, for splitting them over a team)
     // and the coloured non-parallel group (empty when it holds skinned or rod constraints)
     std::vector<WindowDev> par_windows;
+    double streamed_us = 0.0;                   // estimated duration of its windows' task programs (µs per iteration)
     DevBuf<uint4> colour_recs;
     DevBuf<uint32_t> colour_begin;
     uint32_t num_colours = 0;
@@ -192,12 +195,10 @@ struct BundleHost
 {
     std::vector<uint32_t> bodies;
     uint32_t nv = 0;
-    bool staged = false;
     bool uniform = false;
     float inv_mass = 0.0f;
-    uint32_t lds = 0;
-    DevBuf<uint4> recs;
-    DevBuf<uint32_t> lvl;
+    DevBuf<uint4> recs, heads;
+    DevBuf<uint32_t> desc;
     DevBuf<BundleBodyDev> table;
     DevBuf<float4> x, v, prev, plane, report, face_scratch;
     DevBuf<int32_t> idx, contact;
@@ -267,9 +268,8 @@ struct xpbd_context
     uint32_t team_lds = 0, team_max_leaves = 0;
     struct BundleLaunch
     {
-        bool staged = false;    // records staged in LDS (256-thread launches)
         bool uniform = false;   // 12 B LDS positions, one inverse mass per bundle
-        uint32_t block = 256;   // threads per workgroup
+        uint32_t block = 512;   // threads per workgroup
         uint32_t lds = 0;       // LDS bytes per workgroup
         DevBuf<BundleDev> table;
         uint32_t count = 0;
@@ -481,6 +481,146 @@ struct GroupLevels
     std::vector<Item> seq;
     std::vector<std::vector<uint32_t>> levels;
 };
+
+// Builds the task programs the kernels run (TaskStream in xpbd_device.h): per wavefront a list of
+// tasks with their records, per task one descriptor.
+struct TaskProgram
+{
+    std::vector<uint4> recs;        // per wavefront, in task order; one record behind the last
+    std::vector<uint32_t> desc;     // per wavefront, kDescPad zero descriptors behind each list
+    std::vector<uint4> heads;       // per wavefront {first descriptor, tasks, first record, trailing barriers}
+    double ns = 0.0;                // estimated duration of one run
+};
+
+struct TaskBuilder
+{
+    // a step fetches descriptors six tasks ahead and runs three tasks at a time
+    static constexpr uint32_t kDescPad = 12;
+    // Instructions of one projection by type (volume, bend, edge, LRA), on one lane and on four.
+    // A lone wavefront issues one instruction in about 5 cycles and a SIMD one in 4, so a level
+    // takes its longest task or a quarter of all its tasks, whichever is more: narrow levels
+    // run four lanes per constraint, wide ones one.
+    static constexpr double kLaneCost[4] = { 142.0, 290.0, 70.0, 60.0 };
+    static constexpr double kQuadCost[4] = { 93.0, 215.0, 48.0, 60.0 };
+
+    uint32_t waves;
+    double simds;                       // SIMDs this workgroup has to itself
+    std::vector<std::vector<uint4>> wrecs;
+    std::vector<std::vector<uint32_t>> wdesc;
+    std::vector<uint32_t> pending;      // barriers since the wavefront's last task
+    std::vector<double> load;
+    int last_single = -1;               // wavefront that ran the whole previous level alone, or -1
+    double ns = 0.0;
+
+    TaskBuilder(uint32_t w, double s) : waves(w), simds(s), wrecs(w), wdesc(w), pending(w, 0), load(w) {}
+
+    // One level; bucket[type]: its records (each bend once).
+    void Level(const std::vector<uint4> (&bucket)[4])
+    {
+        constexpr double kAlone = 1.15;
+        uint32_t best = 0;
+        double best_cost = 1e300;
+        for (uint32_t m = 0; m < 8; ++m)        // types 0 to 2 that run on four lanes
+        {
+            double longest = 0.0, total = 0.0;
+            bool redundant = false;
+            for (uint32_t t = 0; t < 4; ++t)
+            {
+                const bool quad = t < 3 && ((m >> t) & 1u);
+                if (bucket[t].empty())
+                {
+                    redundant |= quad;
+                    continue;
+                }
+                const size_t per = quad ? 16 : 64, tasks = (bucket[t].size() + per - 1) / per;
+                const double c = quad ? kQuadCost[t] : kLaneCost[t];
+                longest = std::max(longest, c);
+                total += c * (double)tasks;
+            }
+            const double cost = std::max(kAlone * longest, total / simds);
+            if (!redundant && cost < best_cost)
+            {
+                best_cost = cost;
+                best = m;
+            }
+        }
+        size_t tasks = 0;
+        for (uint32_t t = 0; t < 4; ++t)
+        {
+            const size_t per = t < 3 && ((best >> t) & 1u) ? 16 : 64;
+            tasks += (bucket[t].size() + per - 1) / per;
+        }
+        std::fill(load.begin(), load.end(), 0.0);
+        const bool single = tasks == 1;
+        // longest kinds first, each task to the wavefront with the least work in this level
+        uint32_t order[4] = { 1, 0, 2, 3 };
+        std::sort(order, order + 4, [&](uint32_t a, uint32_t b) {
+            const double ca = a < 3 && ((best >> a) & 1u) ? kQuadCost[a] : kLaneCost[a];
+            const double cb = b < 3 && ((best >> b) & 1u) ? kQuadCost[b] : kLaneCost[b];
+            return ca != cb ? ca > cb : a < b;
+        });
+        for (uint32_t t : order)
+        {
+            const bool quad = t < 3 && ((best >> t) & 1u);
+            const size_t per = quad ? 16 : 64;
+            for (size_t o = 0; o < bucket[t].size(); o += per)
+            {
+                const uint32_t n = (uint32_t)std::min(per, bucket[t].size() - o);
+                uint32_t w = 0;
+                if (single && last_single >= 0)
+                {
+                    // the wavefront that ran the previous level alone runs this one too: LDS
+                    // operations of one wavefront are in order, no barrier is needed between them
+                    w = (uint32_t)last_single;
+                    for (uint32_t k = 0; k < waves; ++k) --pending[k];
+                }
+                else
+                    w = (uint32_t)(std::min_element(load.begin(), load.end()) - load.begin());
+                load[w] += quad ? kQuadCost[t] : kLaneCost[t];
+                wdesc[w].push_back(n | ((quad ? 4u + t : t) << 7) | (pending[w] << 10));
+                pending[w] = 0;
+                wrecs[w].insert(wrecs[w].end(), bucket[t].begin() + o, bucket[t].begin() + o + n);
+                if (single)
+                    last_single = (int)w;
+            }
+        }
+        if (!single)
+            last_single = -1;
+        for (uint32_t &p : pending) ++p;
+        ns += 170.0 + 2.25 * (tasks ? best_cost : 0.0);
+    }
+
+    // Appends the program to `out`: its records, descriptors and `waves` heads.
+    void Finish(TaskProgram &out)
+    {
+        for (uint32_t w = 0; w < waves; ++w)
+        {
+            out.heads.push_back(make_uint4((uint32_t)out.desc.size(), (uint32_t)wdesc[w].size(), (uint32_t)out.recs.size(), pending[w]));
+            out.recs.insert(out.recs.end(), wrecs[w].begin(), wrecs[w].end());
+            out.desc.insert(out.desc.end(), wdesc[w].begin(), wdesc[w].end());
+            out.desc.insert(out.desc.end(), kDescPad, 0u);
+        }
+        out.recs.push_back(make_uint4(0u, 0u, 0u, 0u));     // read, not used, behind a task's records
+        out.ns += ns;
+    }
+};
+constexpr double TaskBuilder::kLaneCost[4], TaskBuilder::kQuadCost[4];
+
+// Records [begin, end) of a level program by type, without padding and second halves of bends.
+void LevelBuckets(const std::vector<uint4> &recs, size_t begin, size_t end, std::vector<uint4> (&bucket)[4])
+{
+    for (auto &b : bucket) b.clear();
+    for (size_t r = begin; r < end; ++r)
+    {
+        const uint4 &q = recs[r];
+        if (q.x == kNopRecordHost)
+            continue;
+        const uint32_t t = (q.x >> 14) & 3u;
+        if (t == kTypeBend && (q.y & kSecondHalf))
+            continue;
+        bucket[t].push_back(q);
+    }
+}
 
 // Appends one level: records grouped by constraint type (bend, volume, edge,
 // LRA), each group padded with no-op records to whole wavefronts when that does
@@ -1107,6 +1247,27 @@ int BuildSchedule(const xpbd_settings_desc &d, xpbd_settings &s, int32_t schedul
         s.rods.assign(rods, rods + d.num_rod_stretch_shear);
     }
 
+    // task programs of the gathered windows (bodies with rods run the level programs)
+    if (!resident && d.num_rod_stretch_shear == 0)
+    {
+        TaskProgram tp;
+        std::vector<uint4> bucket[4];
+        for (const WindowDev &w : pb.windows)
+        {
+            TaskBuilder builder(kStreamedWaves, 4.0);
+            for (uint32_t L = 0; L < w.nlev; ++L)
+            {
+                LevelBuckets(pb.recs, pb.lvl[w.lbegin + L], pb.lvl[w.lbegin + L + 1], bucket);
+                builder.Level(bucket);
+            }
+            builder.Finish(tp);
+        }
+        s.streamed_us = 1e-3 * tp.ns;
+        if ((e = s.task_recs.upload(tp.recs)) != hipSuccess || (e = s.task_desc.upload(tp.desc)) != hipSuccess
+            || (e = s.task_heads.upload(tp.heads)) != hipSuccess)
+            return Fail(XPBD_E_DEVICE, std::string("settings upload: ") + hipGetErrorString(e));
+    }
+
     SettingsDev &sd = s.dev;
     sd.rod_const = s.rod_const.p;
     sd.bt_const = s.bt_const.p;
@@ -1114,6 +1275,9 @@ int BuildSchedule(const xpbd_settings_desc &d, xpbd_settings &s, int32_t schedul
     sd.recs = s.recs.p;
     sd.lvl = s.lvl.p;
     sd.windows = s.windows.p;
+    sd.task_recs = s.task_recs.p;
+    sd.task_desc = s.task_desc.p;
+    sd.task_heads = s.task_heads.p;
     sd.vlist = s.vlist.p;
     sd.faces = s.faces.p;
     sd.vf_begin = s.vf_begin.p;
@@ -1130,43 +1294,24 @@ int BuildSchedule(const xpbd_settings_desc &d, xpbd_settings &s, int32_t schedul
 // ------------------------------------------------------------------ bundles
 // Bodies whose positions fit in LDS are packed into bundles that share one
 // workgroup.  Bodies are sorted by the length of their level sequence so a
-// bundle holds bodies of similar depth, then packed greedily while the bundle
-// fits the middle launch class.  The bundle's program merges the bodies' level
-// sequences by index; inside a merged level the records are grouped by
-// constraint type and each group is padded to whole wavefronts when that does
-// not add a pass.
+// bundle holds bodies of similar depth, then packed greedily up to the smaller
+// launch class.  The bundle's program merges the bodies' level sequences by index.
 constexpr uint32_t kBundleMaxBodies = 64;
+// Workgroups of the smaller launch class the chip runs at once: 256 CUs x 2
+constexpr uint32_t kResidentWorkgroups = 512;
 
-// Launch classes of the bundles.  A CU has 160 KB of LDS, so the classes hold
-// 4, 2 and 1 workgroups per CU; their threads per workgroup keep the wavefronts
-// of co-resident workgroups within what the kernel's registers allow (5 per
-// SIMD at its ~86 VGPRs).  Bundles are packed to the middle class; single
-// bodies too large for it take the largest.  A large update runs in two bundle
-// launches plus the streamed bodies' launch, each on a hardware queue of its
-// own; the smallest class only takes bundles whose programs fit in LDS with
-// them (small scenes).
+// Launch classes of the bundles.  A CU has 160 KB of LDS, so the classes hold 2 and 1
+// workgroups per CU, either way 16 wavefronts.  Bundles are packed to the smaller class;
+// single bodies too large for it take the larger.  A large update runs in two bundle
+// launches plus the streamed bodies' launch, each on a hardware queue of its own.
 struct BundleClass { uint32_t lds; uint32_t block; double per_cu; };
-constexpr int kNumBundleClasses = 3;
-constexpr BundleClass kBundleClasses[kNumBundleClasses] = {
-    { 40u * 1024u, 256u, 4.0 }, { 80u * 1024u, 512u, 2.0 }, { kMaxLdsBytes, 1024u, 1.0 } };
+constexpr int kNumBundleClasses = 2;
+constexpr BundleClass kBundleClasses[kNumBundleClasses] = { { 80u * 1024u, 512u, 2.0 }, { kMaxLdsBytes, 1024u, 1.0 } };
 
-// Duration of one level pass (µs) of a workgroup of `block` threads, measured
-// with per-workgroup timestamps on MI355X: the pass is a dependent chain of LDS
-// reads, one projection and LDS writes, then a workgroup barrier.
-double LevelPassMicroseconds(uint32_t block)
-{
-    return block >= 1024u ? 1.06 : block >= 512u ? 0.97 : 0.90;
-}
-
-// Level passes of a program for a workgroup of `block` threads: a level of n
-// records takes ceil(n / block) passes.
-double ProgramPasses(const std::vector<uint32_t> &lvl, uint32_t block)
-{
-    double p = 0.0;
-    for (size_t k = 0; k + 1 < lvl.size(); ++k)
-        p += (double)((lvl[k + 1] - lvl[k] + block - 1) / block);
-    return p;
-}
+// Duration of one level pass (µs) of a streamed body with rods, measured with per-workgroup
+// timestamps on MI355X: a dependent chain of LDS reads, one projection and LDS writes, then a
+// workgroup barrier.
+constexpr double kRodLevelMicroseconds = 1.06;
 
 uint4 OffsetRecord(uint4 r, uint32_t voff, uint32_t skin_base)
 {
@@ -1188,13 +1333,12 @@ uint4 OffsetRecord(uint4 r, uint32_t voff, uint32_t skin_base)
 }
 
 void BuildBundleProgram(const xpbd_context *ctx, const BundleHost &bh, const std::vector<uint32_t> &voffs, uint32_t block,
-                        std::vector<uint4> &recs, std::vector<uint32_t> &lvl)
+                        double simds, TaskProgram &out)
 {
-    recs.clear();
-    lvl.clear();
     size_t K = 0;
     for (uint32_t bi : bh.bodies)
         K = std::max(K, ctx->bodies[bi]->settings->host_level_begin.size() - 1);
+    TaskBuilder builder(block / 64u, simds);
     std::vector<uint4> bucket[4];
     for (size_t k = 0; k < K; ++k)
     {
@@ -1209,15 +1353,14 @@ void BuildBundleProgram(const xpbd_context *ctx, const BundleHost &bh, const std
                 if (st.host_recs[r].x == kNopRecordHost)
                     continue;
                 if (((st.host_recs[r].x >> 14) & 3u) == kTypeBend && (st.host_recs[r].y & kSecondHalf))
-                    continue;       // re-emitted with its first half
+                    continue;
                 uint4 rec = OffsetRecord(st.host_recs[r], voffs[j], ctx->bodies[bh.bodies[j]]->dev.skin_base);
                 bucket[(rec.x >> 14) & 3u].push_back(rec);
             }
         }
-        lvl.push_back((uint32_t)recs.size());
-        AppendTypedLevel(bucket, recs, true, nullptr, nullptr, block);
+        builder.Level(bucket);
     }
-    lvl.push_back((uint32_t)recs.size());
+    builder.Finish(out);
 }
 
 // Estimated duration (µs per collision step) of a streamed body: its gathered
@@ -1225,8 +1368,10 @@ void BuildBundleProgram(const xpbd_context *ctx, const BundleHost &bh, const std
 double StreamedMicroseconds(const Body &b)
 {
     const SettingsDev &sd = b.settings->dev;
-    return (double)(sd.num_levels_total + 2u * (sd.num_par_windows + sd.num_tail_windows)) * (double)b.dev.iterations
-           * LevelPassMicroseconds(1024u);
+    const double windows = 2.0 * (sd.num_par_windows + sd.num_tail_windows);
+    if (b.settings->rods.empty() && !sd.resident)
+        return (b.settings->streamed_us + windows) * (double)b.dev.iterations;
+    return (sd.num_levels_total + windows) * (double)b.dev.iterations * kRodLevelMicroseconds;
 }
 
 // Teams.  A streamed body without rods, pressure, dynamic or sensor colliders runs on a
@@ -1361,19 +1506,15 @@ int BuildLayout(xpbd_context *ctx)
     };
     std::vector<uint32_t> resident;
     ctx->streamed.clear();
-    double critical = 0.0;      // longest estimated duration of a single workgroup (µs per step)
     for (uint32_t i = 0; i < ctx->bodies.size(); ++i)
     {
         const Body &b = *ctx->bodies[i];
-        const bool fits = bundle_lds_bytes(b.nv, 0, 0, 1, b.settings->uniform_mass) <= kMaxLdsBytes;
+        const bool fits = bundle_lds_bytes(b.nv, 1, b.settings->uniform_mass) <= kMaxLdsBytes;
         // rod states stay in global memory: bodies with rods run in the per-body kernel
         if (ctx->use_bundles && fits && !b.settings->host_level_begin.empty() && b.settings->rods.empty())
             resident.push_back(i);
         else
-        {
             ctx->streamed.push_back(i);
-            critical = std::max(critical, StreamedMicroseconds(b));
-        }
     }
     if (int rc = BuildTeams(ctx))
         return rc;
@@ -1389,7 +1530,13 @@ int BuildLayout(xpbd_context *ctx)
         return A.settings->host_level_begin.size() > B.settings->host_level_begin.size();
     });
     std::vector<std::unique_ptr<BundleHost>> bundles;
-    const uint32_t pack_lds = kBundleClasses[1].lds;
+    // Bodies share a workgroup only when there are more of them than the chip holds workgroups
+    // (two per CU): merged levels are wider and take longer, so a small scene spreads its bodies
+    // over the CUs.
+    size_t all_lds = 0;
+    for (uint32_t bi : resident)
+        all_lds += bundle_lds_bytes(ctx->bodies[bi]->nv, 1, uniform_of(bi));
+    const uint32_t pack_lds = (uint32_t)std::min<size_t>(kBundleClasses[0].lds, all_lds / kResidentWorkgroups);
     for (uint32_t bi : resident)
     {
         const Body &b = *ctx->bodies[bi];
@@ -1398,7 +1545,7 @@ int BuildLayout(xpbd_context *ctx)
                                 && (!uniform_of(bi) || mass_bits(cur->bodies[0]) == mass_bits(bi))
                                 && ctx->bodies[cur->bodies[0]]->dev.iterations == b.dev.iterations;
         const bool fits = same_class && cur->bodies.size() < kBundleMaxBodies
-                          && bundle_lds_bytes(cur->nv + b.nv, 0, 0, (uint32_t)cur->bodies.size() + 1u, uniform_of(bi)) <= pack_lds;
+                          && bundle_lds_bytes(cur->nv + b.nv, (uint32_t)cur->bodies.size() + 1u, uniform_of(bi)) <= pack_lds;
         if (!fits)
         {
             bundles.emplace_back(new BundleHost);
@@ -1410,22 +1557,17 @@ int BuildLayout(xpbd_context *ctx)
         cur->nv += b.nv;
     }
 
-    // Programs and launch classes.  Each bundle goes to the class that spends the
-    // fewest CU-microseconds on it (duration / workgroups per CU) without making
-    // it longer than the longest workgroup the update has anyway.
+    // Programs and launch classes: a bundle takes the smallest class its positions fit.
     struct Plan
     {
         std::vector<uint32_t> voffs;
-        std::vector<uint4> recs;
-        std::vector<uint32_t> lvl;
-        double passes[3];       // level passes per iteration at 256, 512, 1024 threads
-        uint32_t plain_lds, staged_lds, iterations, foff;
+        TaskProgram program;
+        uint32_t iterations, foff;
         bool has_pressure, has_sleepers;
         int cls;
-        double us;              // estimated µs per collision step in its class
+        double us;              // estimated µs per collision step
     };
     std::vector<Plan> plans(bundles.size());
-    const uint32_t blocks[3] = { 256u, 512u, 1024u };
     for (size_t k = 0; k < bundles.size(); ++k)
     {
         BundleHost &bh = *bundles[k];
@@ -1451,54 +1593,14 @@ int BuildLayout(xpbd_context *ctx)
         bh.nv = voff;
         P.foff = foff;
         P.iterations = ctx->bodies[bh.bodies[0]]->dev.iterations;
-        BuildBundleProgram(ctx, bh, P.voffs, 256u, P.recs, P.lvl);
-        for (int q = 0; q < 3; ++q)
-            P.passes[q] = ProgramPasses(P.lvl, blocks[q]);
-        const uint32_t nlev = (uint32_t)P.lvl.size() - 1;
-        P.plain_lds = bundle_lds_bytes(voff, 0, 0, nb, bh.uniform);
-        P.staged_lds = bundle_lds_bytes(voff, (uint32_t)P.recs.size(), nlev + 1, nb, bh.uniform);
-        if (P.plain_lds > kMaxLdsBytes)
+        const uint32_t lds = bundle_lds_bytes(voff, nb, bh.uniform);
+        if (lds > kMaxLdsBytes)
             return Fail(XPBD_E_CAPACITY, "bundle needs more LDS than a workgroup has");
-        // shortest duration any class can give this bundle
-        double best = 1e300;
-        for (int q = 0; q < 3; ++q)
-            best = std::min(best, P.iterations * P.passes[q] * LevelPassMicroseconds(blocks[q]));
-        critical = std::max(critical, best);
-    }
-    auto class_block = [&](int c) { return kBundleClasses[c].block; };
-    auto class_us = [&](const Plan &P, int c) {
-        const uint32_t blk = class_block(c);
-        return P.iterations * P.passes[blk == 1024u ? 2 : blk == 512u ? 1 : 0] * LevelPassMicroseconds(blk);
-    };
-    for (Plan &P : plans)
-    {
-        // fewest CU-microseconds among the classes that keep the bundle within the
-        // critical duration; the shortest class when none does
-        P.cls = -1;
-        int fastest = -1;
-        double best_cost = 1e300, fastest_us = 1e300;
-        for (int c = 0; c < kNumBundleClasses; ++c)
-        {
-            // the smallest class is for bundles whose records fit in LDS with them
-            // (small programs): a fourth bundle launch would share a hardware queue
-            if (P.plain_lds > kBundleClasses[c].lds || (c == 0 && P.staged_lds > kBundleClasses[0].lds))
-                continue;
-            const double us = class_us(P, c);
-            if (us < fastest_us)
-            {
-                fastest = c;
-                fastest_us = us;
-            }
-            const double cost = us / kBundleClasses[c].per_cu;
-            if (us <= critical * 1.0001 && cost < best_cost)
-            {
-                P.cls = c;
-                best_cost = cost;
-            }
-        }
-        if (P.cls < 0)
-            P.cls = fastest;
-        P.us = class_us(P, P.cls);
+        P.cls = lds <= kBundleClasses[0].lds ? 0 : 1;
+        // workgroups that share a CU share its four SIMDs
+        const double simds = P.cls == 0 && bundles.size() > kResidentWorkgroups / 2u ? 2.0 : 4.0;
+        BuildBundleProgram(ctx, bh, P.voffs, kBundleClasses[P.cls].block, simds, P.program);
+        P.us = 1e-3 * P.program.ns * P.iterations;
     }
 
     HIP_TRY(ctx->d_elapsed.alloc(std::max<size_t>(1, bundles.size())));
@@ -1512,17 +1614,15 @@ int BuildLayout(xpbd_context *ctx)
         ctx->h_elapsed_n = bundles.size();
     }
     ctx->order_state = xpbd_context::kOrderMeasure;
-    // one launch per class and LDS layout (staged records, 12 B positions): slot 4 class + 2 staged + uniform
-    std::vector<std::unique_ptr<xpbd_context::BundleLaunch>> launches(4 * kNumBundleClasses);
-    std::vector<std::vector<std::pair<double, BundleDev>>> launch_tables(4 * kNumBundleClasses);
+    // one launch per class and LDS layout (12 B positions): slot 2 class + uniform
+    std::vector<std::unique_ptr<xpbd_context::BundleLaunch>> launches(2 * kNumBundleClasses);
+    std::vector<std::vector<std::pair<double, BundleDev>>> launch_tables(2 * kNumBundleClasses);
     for (size_t k = 0; k < bundles.size(); ++k)
     {
         BundleHost &bh = *bundles[k];
         Plan &P = plans[k];
         const uint32_t nb = (uint32_t)bh.bodies.size();
-        const uint32_t block = class_block(P.cls);
-        if (block != 256u)
-            BuildBundleProgram(ctx, bh, P.voffs, block, P.recs, P.lvl);
+        const uint32_t block = kBundleClasses[P.cls].block;
         std::vector<BundleBodyDev> table(nb);
         uint32_t foff = 0;
         for (uint32_t j = 0; j < nb; ++j)
@@ -1533,8 +1633,9 @@ int BuildLayout(xpbd_context *ctx)
                 foff += b.settings->num_faces;
         }
         const uint32_t voff = bh.nv;
-        HIP_TRY(bh.recs.upload(P.recs));
-        HIP_TRY(bh.lvl.upload(P.lvl));
+        HIP_TRY(bh.recs.upload(P.program.recs));
+        HIP_TRY(bh.desc.upload(P.program.desc));
+        HIP_TRY(bh.heads.upload(P.program.heads));
         HIP_TRY(bh.table.upload(table));
         // bundle-contiguous vertex state, gathered from wherever each body's state lives now
         HIP_TRY(bh.x.alloc(voff)); HIP_TRY(bh.v.alloc(voff)); HIP_TRY(bh.prev.alloc(voff)); HIP_TRY(bh.plane.alloc(voff));
@@ -1556,7 +1657,7 @@ int BuildLayout(xpbd_context *ctx)
         HIP_TRY(bh.leaves.alloc((size_t)std::max(1u, nb * nc) * bundle_leaf_bytes()));
         HIP_TRY(bh.face_scratch.alloc(std::max(1u, P.foff)));
         BundleDev &d = bh.dev;
-        d.recs = bh.recs.p; d.lvl = bh.lvl.p; d.nlev = (uint32_t)P.lvl.size() - 1; d.num_records = (uint32_t)P.recs.size();
+        d.recs = bh.recs.p; d.desc = bh.desc.p; d.heads = bh.heads.p;
         d.bodies = bh.table.p; d.num_bodies = nb; d.nv = voff;
         d.x = bh.x.p; d.v = bh.v.p; d.prev = bh.prev.p; d.plane = bh.plane.p; d.idx = bh.idx.p; d.contact = bh.contact.p;
         d.report = bh.report.p;
@@ -1568,15 +1669,10 @@ int BuildLayout(xpbd_context *ctx)
         d.uniform_inv_mass = bh.uniform ? bh.inv_mass : 0.0f;
         d.elapsed = ctx->d_elapsed.p + k;
         d.skin = ctx->d_skin.p;
-        // records staged in LDS when the bundle still fits the smallest class with them
-        bh.staged = block == 256u && bundle_lds_bytes(voff, d.num_records, d.nlev + 1, nb, bh.uniform) <= kBundleClasses[0].lds;
-        d.staged = bh.staged ? 1u : 0u;
-        bh.lds = kBundleClasses[P.cls].lds;
-        const int slot = 4 * P.cls + (bh.staged ? 2 : 0) + (bh.uniform ? 1 : 0);
+        const int slot = 2 * P.cls + (bh.uniform ? 1 : 0);
         if (!launches[slot])
         {
             launches[slot].reset(new xpbd_context::BundleLaunch);
-            launches[slot]->staged = bh.staged;
             launches[slot]->uniform = bh.uniform;
             launches[slot]->block = block;
             launches[slot]->lds = kBundleClasses[P.cls].lds;
@@ -1606,7 +1702,7 @@ int BuildLayout(xpbd_context *ctx)
     // starts before smaller workgroups take parts of every CU.  Inside a launch the
     // longest bundles come first (workgroups are dispatched in index order).
     ctx->bundle_launches.clear();
-    for (int c = 4 * kNumBundleClasses - 1; c >= 0; --c)
+    for (int c = 2 * kNumBundleClasses - 1; c >= 0; --c)
     {
         if (!launches[c])
             continue;
@@ -2546,7 +2642,7 @@ int xpbd_update(xpbd_context *ctx, float dt, int32_t collision_steps, int32_t fr
         const auto &L = *Lp;
         const int best = least_queued();
         queued[best] += std::max(L.cost, L.work / 256.0);
-        HIP_TRY(launch_bundles(L.staged, L.block, L.uniform, ctx->ext_colliders, L.table.p, L.count, ctx->d_bodies.p, ctx->d_states.p, ctx->d_colliders.p, nc,
+        HIP_TRY(launch_bundles(L.block, L.uniform, ctx->ext_colliders, L.table.p, L.count, ctx->d_bodies.p, ctx->d_states.p, ctx->d_colliders.p, nc,
                                L.lds, gx, gy, gz, dt, collision_steps, frames, streams[best]));
     }
     for (int a = 0; a < num_aux; ++a)

@@ -21,6 +21,9 @@ enum : uint32_t { kTypeVolume = 0, kTypeBend = 1, kTypeEdge = 2, kTypeLRA = 3 };
 constexpr uint32_t kRodStretchShear = 0x80000000u, kRodBendTwist = 0x40000000u, kRodIndexMask = 0x3fffffffu;
 constexpr uint32_t kMaxWindowVertices = 1u << 14;
 
+// Wavefronts of a workgroup that runs a streamed body or a team member (1024 threads)
+constexpr uint32_t kStreamedWaves = 16;
+
 // A window is a set of vertices held in LDS while a run of levels executes on
 // it.  Resident bodies keep all their vertices in LDS for the whole launch and
 // use identity windows (vcount == 0: record vertex numbers are body vertex
@@ -37,6 +40,11 @@ struct SettingsDev
     const uint4 *recs;          // records ordered (window, level)
     const uint32_t *lvl;        // absolute record offset of each level start, nlev+1 per window
     const WindowDev *windows;   // parallel-group windows, then tail windows
+    // gathered windows without rods run as task programs of kStreamedWaves wavefronts: records,
+    // descriptors, and kStreamedWaves heads per window
+    const uint4 *task_recs;
+    const uint32_t *task_desc;
+    const uint4 *task_heads;
     const uint32_t *vlist;      // gathered windows' vertex lists (body vertex indices)
     const uint32_t *faces;      // 3 vertex indices per face (pressure)
     const uint32_t *vf_begin;   // vertex -> face CSR, faces in increasing order (pressure)
@@ -220,8 +228,8 @@ namespace xpbd {
 // A bundle is a set of LDS-resident bodies that share one workgroup.  Each
 // body's level sequence (merged parallel-group levels, then the non-parallel
 // group's levels) is merged with the others' by index, so level k of every
-// body runs in one barrier-separated pass; within a level the records are
-// grouped by constraint type and padded to whole wavefronts.
+// body runs in one barrier-separated pass, as a task program of the workgroup's
+// wavefronts.
 struct BundleBodyDev
 {
     uint32_t body;              // index into the context's body table
@@ -232,10 +240,9 @@ struct BundleBodyDev
 
 struct BundleDev
 {
-    const uint4 *recs;          // merged level program (vertex numbers are bundle-local)
-    const uint32_t *lvl;        // nlev + 1 absolute record offsets
-    uint32_t nlev;
-    uint32_t num_records;
+    const uint4 *recs;          // task program of the merged levels (vertex numbers are bundle-local)
+    const uint32_t *desc;
+    const uint4 *heads;         // one per wavefront
     const BundleBodyDev *bodies;
     uint32_t num_bodies;
     uint32_t nv;                // vertices of all bodies of the bundle
@@ -247,7 +254,6 @@ struct BundleDev
     uint32_t has_pressure;
     uint32_t has_sleepers;
     uint32_t iterations;
-    uint32_t staged;            // records + level offsets copied into LDS once per launch (256-thread launches)
     uint32_t uniform;           // 12 B LDS positions: every vertex has the inverse mass uniform_inv_mass
     float uniform_inv_mass;
     unsigned long long *elapsed;    // where the workgroup stores its duration (realtime-clock ticks), or null
