@@ -383,12 +383,12 @@ __device__ __forceinline__ void bundle_update(
 
                 // ---- merged level program of all bodies (skin records carry their entries)
                 const RecordCtx sk{ G.skin, 0u, (float)(it + 1) / (float)iterations };
-                TaskStream tasks;
+                TaskStream<> tasks;
                 tasks.begin(G.recs, G.desc, G.heads + wave, lane);
                 if (has_sleepers)
-                    tasks.run(X, inv_dt_sq, lane, [&](const uint4 &r) { return !st[vb[r.x & 0x3fffu]].active; }, sk);
+                    run_tasks(tasks, X, inv_dt_sq, lane, [&](const uint4 &r) { return !st[vb[r.x & 0x3fffu]].active; }, sk);
                 else
-                    tasks.run(X, inv_dt_sq, lane, NoSkip(), sk);
+                    run_tasks(tasks, X, inv_dt_sq, lane, NoSkip(), sk);
 
                 // ---- collision + velocity (SoftBodyMotionProperties.cpp:700-825), fused with the
                 // next integration (no pressure) or the per-vertex part of UpdateSoftBodyState.

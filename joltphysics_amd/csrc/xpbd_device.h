@@ -396,14 +396,15 @@ __device__ __forceinline__ float cget(const PositionsF3 &X, uint32_t i, uint32_t
 __device__ __forceinline__ float wget(const PositionsF3 &X, uint32_t) { return X.w; }
 __device__ __forceinline__ void cset(const PositionsF3 &X, uint32_t i, uint32_t c, float v) { X.x[3u * i + c] = v; }
 
+// (delta, length: the difference of the positions before the projection, and its length)
 template <class P>
 __device__ __forceinline__ void project_edge_quad(const P &X, uint32_t c, uint32_t i0, uint32_t i1, float rest, float compliance,
-                                                  float inv_dt_sq)
+                                                  float inv_dt_sq, float &delta, float &length)
 {
     const float x0 = cget(X, i0, c), x1 = cget(X, i1, c);
     const float w0 = wget(X, i0), w1 = wget(X, i1);
-    const float delta = x1 - x0;
-    const float length = square_root(quad_dot(delta, delta));
+    delta = x1 - x0;
+    length = square_root(quad_dot(delta, delta));
     const float denom = length * ((w0 + w1) + compliance * inv_dt_sq);
     const float correction = (delta * (length - rest)) / denom;
     if (!(denom < 1.0e-12f))
@@ -779,43 +780,66 @@ __device__ __forceinline__ void run_levels_global(const uint4 *recs, const uint3
 enum TaskKind : uint32_t { kTaskVolume = 0, kTaskBend = 1, kTaskEdge = 2, kTaskLRA = 3, kTaskVolumeQuad = 4, kTaskBendQuad = 5, kTaskEdgeQuad = 6 };
 constexpr uint32_t kTaskQuadBit = 4u << 7;
 
+// Per-task data a program loads ahead besides the records (see TaskStream)
+struct NoAux
+{
+    struct Value {};
+    __device__ __forceinline__ Value load(uint32_t, uint32_t, uint32_t) const { return Value{}; }
+};
+
+// REVERSE runs the tasks backwards (the adjoint of a program); the caller synchronises the
+// workgroup after a reverse run, whose last level no barrier follows.  aux.load(record, descriptor,
+// lane) is loaded with the records, three tasks ahead; handle(descriptor, record, aux value,
+// index of the task's first record) projects one task.
+template <bool REVERSE = false, class Aux = NoAux>
 struct TaskStream
 {
-    const uint4 *recs;          // next record to fetch
+    const uint4 *recs;
+    uint32_t pos;               // record index of the next task to fetch (forward), or behind it (reverse)
     const uint32_t *desc;
     uint32_t desc_offset;       // byte offset of the next descriptor (the same in every lane)
     uint32_t count, trail;
-    uint32_t d0, d1, d2;        // descriptors of the fetched records (uniform)
-    uint32_t q0, q1, q2;        // the next three descriptors
+    uint32_t d0, d1, d2, p0, p1, p2;    // descriptors and record indices of the fetched tasks (uniform)
+    uint32_t q0, q1, q2;                // the next three descriptors
     RecordVec r0, r1, r2;
+    typename Aux::Value a0, a1, a2;
 
     __device__ __forceinline__ uint32_t next_desc()
     {
-        const uint32_t v = *(const __attribute__((address_space(1))) uint32_t *)(const void *)((const char *)desc + desc_offset);
-        desc_offset += 4u;
+        const uint32_t v = *(const __attribute__((address_space(1))) uint32_t *)(const void *)((const char *)desc + (int32_t)desc_offset);
+        desc_offset += REVERSE ? (uint32_t)-4 : 4u;
         return v;
     }
     // the record of this lane, or the one behind the task's last
-    __device__ __forceinline__ RecordVec fetch(uint32_t d, uint32_t lane)
+    __device__ __forceinline__ RecordVec fetch(uint32_t d, uint32_t lane, uint32_t &p, typename Aux::Value &a, const Aux &aux)
     {
         const uint32_t n = d & 127u;
         const uint32_t i = (d & kTaskQuadBit) ? lane >> 2 : lane;
-        const RecordVec r = load_record(recs, i < n ? i : n);
-        recs += n;
+        if (REVERSE)
+            pos -= n;
+        p = pos;
+        const RecordVec r = load_record(recs + pos, i < n ? i : n);
+        a = aux.load(p + (i < n ? i : 0u), d, lane);
+        if (!REVERSE)
+            pos += n;
         return r;
     }
-    // `head`: {first descriptor, tasks, first record, barriers after the last task} of this wavefront.
-    // Issues the first loads; the caller may do other work before run().
-    __device__ __forceinline__ void begin(const uint4 *all_recs, const uint32_t *all_desc, const uint4 *head, uint32_t lane)
+    // `head`: {first descriptor, tasks, first record, barriers after the last task} of this
+    // wavefront, the next wavefront's head behind it.  Issues the first loads; the caller may do
+    // other work before run().
+    __device__ __forceinline__ void begin(const uint4 *all_recs, const uint32_t *all_desc, const uint4 *head, uint32_t lane,
+                                          const Aux &aux = Aux())
     {
         // global stores of an earlier phase still pending would make every later wait a full one
         __builtin_amdgcn_s_waitcnt(kWaitVmcntZero);
-        head = uniform_ptr(head);
-        const uint32_t first = load_level_offset(reinterpret_cast<const uint32_t *>(head), 0);
-        count = load_level_offset(reinterpret_cast<const uint32_t *>(head), 1);
-        recs = uniform_ptr(all_recs) + load_level_offset(reinterpret_cast<const uint32_t *>(head), 2);
-        trail = load_level_offset(reinterpret_cast<const uint32_t *>(head), 3);
-        desc = uniform_ptr(all_desc) + first;
+        const uint32_t *h = reinterpret_cast<const uint32_t *>(uniform_ptr(head));
+        const uint32_t first = load_level_offset(h, 0);
+        count = load_level_offset(h, 1);
+        pos = load_level_offset(h, REVERSE ? 6 : 2);
+        trail = load_level_offset(h, 3);
+        recs = uniform_ptr(all_recs);
+        // signed: a wavefront without tasks starts its reverse run one descriptor before its list
+        desc = uniform_ptr(all_desc) + ((int64_t)first + (REVERSE ? (int64_t)count - 1 : 0));
         desc_offset = 0u;
         asm volatile("" : "+v"(desc_offset));       // a vector register: the loads stay vector loads
         const uint32_t f0 = next_desc(), f1 = next_desc(), f2 = next_desc();
@@ -825,65 +849,90 @@ struct TaskStream
         d0 = uniform(f0);
         d1 = uniform(f1);
         d2 = uniform(f2);
-        r0 = fetch(d0, lane);
+        r0 = fetch(d0, lane, p0, a0, aux);
         asm volatile("" ::: "memory");
-        r1 = fetch(d1, lane);
+        r1 = fetch(d1, lane, p1, a1, aux);
         asm volatile("" ::: "memory");
-        r2 = fetch(d2, lane);
+        r2 = fetch(d2, lane, p2, a2, aux);
     }
-    template <class P, class Skip>
-    __device__ __forceinline__ void step(uint32_t &d, RecordVec &r, uint32_t &q, const P &X, float inv_dt_sq, uint32_t lane, Skip skip,
-                                         const RecordCtx &sk)
+    static __device__ __forceinline__ void barriers(uint32_t n)
     {
-        for (uint32_t k = d >> 10; k > 0; --k)
+        for (; n > 0; --n)
             __syncthreads();
+    }
+    template <class Handle>
+    __device__ __forceinline__ void step(uint32_t &d, RecordVec &r, uint32_t &q, uint32_t &p, typename Aux::Value &a, uint32_t lane,
+                                         Handle handle, const Aux &aux)
+    {
+        if (!REVERSE)
+            barriers(d >> 10);
         pin_record(r);
-        const uint32_t n = d & 127u, kind = (d >> 7) & 7u;
-        const uint32_t i0 = r.x & 0x3fffu, i1 = r.x >> 16, i2 = r.y & 0x3fffu, i3 = r.y >> 16;
-        const float p0 = __uint_as_float(r.z), p1 = __uint_as_float(r.w);
-        if (d & kTaskQuadBit)
-        {
-            if ((lane >> 2) < n && !skip(as_uint4(r)))
-            {
-                const uint32_t c = (lane & 3u) < 2u ? (lane & 3u) : 2u;
-                if (kind == kTaskBendQuad)
-                    project_bend_quad(X, c, i0, i1, i2, i3, p0, p1, inv_dt_sq);
-                else if (kind == kTaskEdgeQuad)
-                    project_edge_quad(X, c, i0, i1, p0, p1, inv_dt_sq);
-                else
-                    project_volume_quad(X, c, i0, i1, i2, i3, p0, p1, inv_dt_sq);
-            }
-        }
-        else if (lane < n && !skip(as_uint4(r)))
-        {
-            if (kind == kTaskEdge)
-                project_edge_wide(X, i0, i1, p0, p1, inv_dt_sq);
-            else if (kind == kTaskBend)
-                project_bend_wide(X, i0, i1, i2, i3, p0, p1, inv_dt_sq);
-            else if (kind == kTaskVolume)
-                project_volume(X, i0, i1, i2, i3, p0, p1, inv_dt_sq);
-            else if (i0 == i1)
-                project_skin(X, i0, r.y + sk.base, p0, p1, sk);
-            else
-                project_lra(X, i0, i1, p0);
-        }
+        handle(d, as_uint4(r), a, p);
+        if (REVERSE)
+            barriers(d >> 10);
         d = uniform(q);
         q = next_desc();
-        r = fetch(d, lane);
+        r = fetch(d, lane, p, a, aux);
     }
-    template <class P, class Skip>
-    __device__ __forceinline__ void run(const P &X, float inv_dt_sq, uint32_t lane, Skip skip, const RecordCtx &sk)
+    template <class Handle>
+    __device__ __forceinline__ void run(uint32_t lane, Handle handle, const Aux &aux = Aux())
     {
+        if (REVERSE)
+            barriers(trail);
         for (uint32_t t = 0; t < count; t += 3)
         {
-            step(d0, r0, q0, X, inv_dt_sq, lane, skip, sk);
-            step(d1, r1, q1, X, inv_dt_sq, lane, skip, sk);
-            step(d2, r2, q2, X, inv_dt_sq, lane, skip, sk);
+            step(d0, r0, q0, p0, a0, lane, handle, aux);
+            step(d1, r1, q1, p1, a1, lane, handle, aux);
+            step(d2, r2, q2, p2, a2, lane, handle, aux);
         }
-        for (uint32_t k = trail; k > 0; --k)
-            __syncthreads();
+        if (!REVERSE)
+            barriers(trail);
     }
 };
+
+// Projects one task on the positions X; skip(record): lanes that leave their constraint out
+template <class P, class Skip>
+__device__ __forceinline__ void project_task(const P &X, uint32_t d, const uint4 &r, float inv_dt_sq, uint32_t lane, Skip skip,
+                                             const RecordCtx &sk)
+{
+    const uint32_t n = d & 127u, kind = (d >> 7) & 7u;
+    const uint32_t i0 = r.x & 0x3fffu, i1 = r.x >> 16, i2 = r.y & 0x3fffu, i3 = r.y >> 16;
+    const float p0 = __uint_as_float(r.z), p1 = __uint_as_float(r.w);
+    if (d & kTaskQuadBit)
+    {
+        if ((lane >> 2) < n && !skip(r))
+        {
+            const uint32_t c = (lane & 3u) < 2u ? (lane & 3u) : 2u;
+            if (kind == kTaskBendQuad)
+                project_bend_quad(X, c, i0, i1, i2, i3, p0, p1, inv_dt_sq);
+            else if (kind == kTaskEdgeQuad)
+            {
+                float delta, length;
+                project_edge_quad(X, c, i0, i1, p0, p1, inv_dt_sq, delta, length);
+            }
+            else
+                project_volume_quad(X, c, i0, i1, i2, i3, p0, p1, inv_dt_sq);
+        }
+    }
+    else if (lane < n && !skip(r))
+    {
+        if (kind == kTaskEdge)
+            project_edge_wide(X, i0, i1, p0, p1, inv_dt_sq);
+        else if (kind == kTaskBend)
+            project_bend_wide(X, i0, i1, i2, i3, p0, p1, inv_dt_sq);
+        else if (kind == kTaskVolume)
+            project_volume(X, i0, i1, i2, i3, p0, p1, inv_dt_sq);
+        else if (i0 == i1)
+            project_skin(X, i0, r.y + sk.base, p0, p1, sk);
+        else
+            project_lra(X, i0, i1, p0);
+    }
+}
+template <class P, class Skip>
+__device__ __forceinline__ void run_tasks(TaskStream<> &tasks, const P &X, float inv_dt_sq, uint32_t lane, Skip skip, const RecordCtx &sk)
+{
+    tasks.run(lane, [&](uint32_t d, const uint4 &r, NoAux::Value, uint32_t) { project_task(X, d, r, inv_dt_sq, lane, skip, sk); });
+}
 
 // Level program with records and offsets in LDS: the first record of the next
 // level is read before the barrier (the barrier's LDS wait covers it).

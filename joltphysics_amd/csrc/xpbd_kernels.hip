@@ -423,9 +423,9 @@ __global__ __launch_bounds__(kBlock) void update_kernel(
                 for (uint32_t w = 0; w < num_windows; ++w)
                 {
                     const WindowDev W = S.windows[w];
-                    TaskStream tasks;
+                    TaskStream<> tasks;
                     if (!RESIDENT && !RODS)
-                        tasks.begin(S.task_recs, S.task_desc, S.task_heads + (size_t)w * kStreamedWaves + wave, (uint32_t)lane);
+                        tasks.begin(S.task_recs, S.task_desc, S.task_heads + (size_t)w * (kStreamedWaves + 1u) + wave, (uint32_t)lane);
                     if (!RESIDENT && W.vcount)
                     {
                         for (uint32_t j = tid; j < W.vcount; j += kBlock)
@@ -434,7 +434,7 @@ __global__ __launch_bounds__(kBlock) void update_kernel(
                     }
                     const RecordCtx rc{ B.skin, B.skin_base, (float)(it + 1) / (float)iterations, B.rods, S.rod_const, S.bt_const };
                     if (!RESIDENT && !RODS)
-                        tasks.run(X, inv_dt_sq, (uint32_t)lane, NoSkip(), rc);
+                        run_tasks(tasks, X, inv_dt_sq, (uint32_t)lane, NoSkip(), rc);
                     else
                         run_levels<STAGED, kBlock, RODS>(recs, lvl + W.lbegin, W.nlev, X, inv_dt_sq, tid, rc, has_rods);
                     if (!RESIDENT && W.vcount)

@@ -29,7 +29,11 @@
 
 namespace xpbd {
 
-constexpr int kRolloutBlock = 256;
+// Threads per workgroup.  Narrow levels leave most wavefronts of a large workgroup idle, but the
+// per-vertex phases and the wide first levels gain more from 16 wavefronts; a body with dihedral
+// bends takes 4, whose adjoint on dual numbers in double needs more registers than 16 leave.
+constexpr int kRolloutBlock = 1024, kRolloutBendBlock = 256;
+constexpr int kRolloutDoubleBlock = 256;
 
 template <class T> struct R3 { T x, y, z; };
 template <class T> struct alignas(sizeof(T) * 4) R4 { T x, y, z, w; };
@@ -114,16 +118,16 @@ __device__ __forceinline__ void lra_project(R4<T> *X, uint32_t i0, uint32_t i1, 
         X[i1] = r4(x0 + (delta * max_distance) / rsqrt_exact(delta_len_sq), p1.w);
 }
 
-// Adjoint of lra_project from its pre-projection positions q0, q1: when the constraint acts,
+// Adjoint of lra_project from t = {delta, |delta|^2} before the projection: when the constraint acts,
 // x1' = x0 + m u with u = delta / |delta|, so with a1 = x1'bar
 //   x1bar = (m / |delta|) (a1 - u (u . a1)),  x0bar = x0'bar + a1 - x1bar.
 // Vertex 0 is only read in the forward pass, so the LRAs of one level may share it (all LRAs
 // of a pinned corner do): their x0bar terms are added atomically.  Nothing else of the level
 // touches it.
-__device__ __forceinline__ void lra_adjoint(float4 *A, uint32_t i0, uint32_t i1, float4 q0, float4 q1, float max_distance)
+__device__ __forceinline__ void lra_adjoint(float4 *A, uint32_t i0, uint32_t i1, const float4 &t, float max_distance)
 {
-    const R3<float> delta = r3(q1.x - q0.x, q1.y - q0.y, q1.z - q0.z);
-    const float delta_len_sq = rdot(delta, delta);
+    const R3<float> delta = r3(t.x, t.y, t.z);
+    const float delta_len_sq = t.w;
     if (!(delta_len_sq > max_distance * max_distance))
         return;
     const float length = sqrtf(delta_len_sq);
@@ -250,41 +254,40 @@ __device__ __forceinline__ void bend_project(R4<T> *X, uint32_t i0, uint32_t i1,
             X[idx[k]] = r4(y[k], X[idx[k]].w);
 }
 
-// Adjoint of bend_project from its pre-projection positions q[4]: xbar = J^T ybar, the
-// Jacobian J of the projection taken one input component at a time on duals.  The Jacobian is
-// evaluated in double at the float positions: near a flat hinge the derivative of
-// ACosApproximate, 1 / (2 sqrt(1 - |x|)), magnifies the rounding of 1 - |x| and float duals lose
-// a few digits there.
-__device__ __forceinline__ void bend_adjoint(float4 *A, uint32_t i0, uint32_t i1, uint32_t i2, uint32_t i3, const float4 *q,
-                                             float compliance, float initial_angle, float inv_dt_sq)
+// Adjoint of a dihedral bend from its pre-projection positions x (float), on a quad of lanes:
+// xbar = J^T ybar, the Jacobian J of the projection taken one input component at a time on duals;
+// lane k takes the three components of vertex k and stores its adjoint.  The Jacobian is evaluated
+// in double at the float positions: near a flat hinge the derivative of ACosApproximate,
+// 1 / (2 sqrt(1 - |x|)), magnifies the rounding of 1 - |x| and float duals lose a few digits there.
+__device__ __forceinline__ void bend_adjoint(float4 *A, uint32_t lane, uint32_t i0, uint32_t i1, uint32_t i2, uint32_t i3,
+                                             const float4 &tx, const float4 &ty, const float4 &tz, float compliance,
+                                             float initial_angle, float inv_dt_sq)
 {
-    const uint32_t idx[4] = { i0, i1, i2, i3 };
-    float w[4];
-    R3<float> ybar[4];
-    for (int k = 0; k < 4; ++k)
-    {
-        w[k] = q[k].w;
-        const float4 a = A[idx[k]];
-        ybar[k] = r3(a.x, a.y, a.z);
-    }
-    double xbar[12];
-    for (int col = 0; col < 12; ++col)
+    const uint32_t own = lane & 3u;
+    const float px[4] = { tx.x, tx.y, tx.z, tx.w }, py[4] = { ty.x, ty.y, ty.z, ty.w }, pz[4] = { tz.x, tz.y, tz.z, tz.w };
+    const float4 ybar[4] = { A[i0], A[i1], A[i2], A[i3] };
+    const float w[4] = { ybar[0].w, ybar[1].w, ybar[2].w, ybar[3].w };
+    double xbar[3];
+#pragma unroll 1
+    for (uint32_t j = 0; j < 3; ++j)
     {
         R3<Dual<double>> x[4], y[4];
-        for (int k = 0; k < 4; ++k)
-            x[k] = r3(dual((double)q[k].x, col == 3 * k ? 1.0 : 0.0), dual((double)q[k].y, col == 3 * k + 1 ? 1.0 : 0.0),
-                      dual((double)q[k].z, col == 3 * k + 2 ? 1.0 : 0.0));
+#pragma unroll
+        for (uint32_t k = 0; k < 4; ++k)
+            x[k] = r3(dual((double)px[k], own == k && j == 0 ? 1.0 : 0.0), dual((double)py[k], own == k && j == 1 ? 1.0 : 0.0),
+                      dual((double)pz[k], own == k && j == 2 ? 1.0 : 0.0));
         bend_generic<Dual<double>, double>(x, w, compliance, initial_angle, (double)inv_dt_sq, y);
         double acc = 0.0;
-        for (int k = 0; k < 4; ++k)
+#pragma unroll
+        for (uint32_t k = 0; k < 4; ++k)
             acc += (y[k].x.d * (double)ybar[k].x + y[k].y.d * (double)ybar[k].y) + y[k].z.d * (double)ybar[k].z;
-        xbar[col] = acc;
+        xbar[0] = j == 0 ? acc : xbar[0];
+        xbar[1] = j == 1 ? acc : xbar[1];
+        xbar[2] = j == 2 ? acc : xbar[2];
     }
-    for (int k = 0; k < 4; ++k)
-    {
-        const float4 a = A[idx[k]];
-        A[idx[k]] = make_float4((float)xbar[3 * k], (float)xbar[3 * k + 1], (float)xbar[3 * k + 2], a.w);
-    }
+    const uint32_t i = own == 0 ? i0 : own == 1 ? i1 : own == 2 ? i2 : i3;
+    const float wi = own == 0 ? w[0] : own == 1 ? w[1] : own == 2 ? w[2] : w[3];
+    A[i] = make_float4((float)xbar[0], (float)xbar[1], (float)xbar[2], wi);
 }
 
 // Record type: 1 for a dihedral bend, whose second-lane half (bit 15 of the second word) the
@@ -314,75 +317,79 @@ __device__ __forceinline__ void volume_project(R4<T> *X, uint32_t i1, uint32_t i
     X[i4] = r4(x4 - (minus_lambda * w4) * d4c, w4);
 }
 
-// Adjoint of volume_project from its pre-projection positions q1..q4 (outputs y_i = x_i - mu w_i d_i,
+// Adjoint of a volume constraint from its pre-projection positions x_1..x_4 (outputs y_i = x_i - mu w_i d_i,
 // mu = c / D, c = |6V| - 6V0, D = sum w_i |d_i|^2 + alpha / h^2, d_i = grad_i 6V):
 //   s = sum w_i d_i . ybar_i,  mubar = -s,  cbar = mubar / D,  Dbar = -mubar mu / D,
 //   dbar_i = -mu w_i ybar_i + 2 w_i Dbar d_i,  xbar_j = ybar_j + cbar sign(6V) d_j, and dbar_i back
 //   through the cross products that form d_i (for a x b: abar = b x dbar, bbar = dbar x a).
-// The volume's compliance is not a parameter of the rollout.
-__device__ __forceinline__ void volume_adjoint(float4 *A, uint32_t i1, uint32_t i2, uint32_t i3, uint32_t i4, const float4 *q,
+// The volume's compliance is not a parameter of the rollout.  On a quad of lanes, component k of
+// every vector per lane (x: this component of the four positions).
+__device__ __forceinline__ void volume_adjoint(float4 *A, uint32_t k, uint32_t i1, uint32_t i2, uint32_t i3, uint32_t i4, const float4 &x,
                                                float six_rest_volume, float compliance, float inv_dt_sq)
 {
-    const R3<float> x1 = xyz3(to_r4<float>(q[0])), x2 = xyz3(to_r4<float>(q[1])), x3 = xyz3(to_r4<float>(q[2])),
-                    x4 = xyz3(to_r4<float>(q[3]));
-    const float w1 = q[0].w, w2 = q[1].w, w3 = q[2].w, w4 = q[3].w;
-    const R3<float> x1x2 = x2 - x1, x1x3 = x3 - x1, x1x4 = x4 - x1, x2x4 = x4 - x2, x2x3 = x3 - x2;
-    const float six = rdot(rcross(x1x2, x1x3), x1x4);
+    const float w1 = wget(A, i1), w2 = wget(A, i2), w3 = wget(A, i3), w4 = wget(A, i4);
+    const float x1x2 = x.y - x.x, x1x3 = x.z - x.x, x1x4 = x.w - x.x, x2x4 = x.w - x.y, x2x3 = x.z - x.y;
+    const float d1 = quad_cross(x2x4, x2x3), d2 = quad_cross(x1x3, x1x4), d3 = quad_cross(x1x4, x1x2), d4 = quad_cross(x1x2, x1x3);
+    const float six = quad_dot(d4, x1x4);
     const float c = fabsf(six) - six_rest_volume;
-    const R3<float> d1 = rcross(x2x4, x2x3), d2 = rcross(x1x3, x1x4), d3 = rcross(x1x4, x1x2), d4 = rcross(x1x2, x1x3);
-    const float denom = (((w1 * rdot(d1, d1) + w2 * rdot(d2, d2)) + w3 * rdot(d3, d3)) + w4 * rdot(d4, d4)) + compliance * inv_dt_sq;
-    if (denom < 1.0e-12f)
-        return;
+    const float denom = (((w1 * quad_dot(d1, d1) + w2 * quad_dot(d2, d2)) + w3 * quad_dot(d3, d3)) + w4 * quad_dot(d4, d4)) + compliance * inv_dt_sq;
     const float mu = c / denom;
-    const float4 a1 = A[i1], a2 = A[i2], a3 = A[i3], a4 = A[i4];
-    const R3<float> y1 = xyz3(to_r4<float>(a1)), y2 = xyz3(to_r4<float>(a2)), y3 = xyz3(to_r4<float>(a3)), y4 = xyz3(to_r4<float>(a4));
-    const float s = ((w1 * rdot(d1, y1) + w2 * rdot(d2, y2)) + w3 * rdot(d3, y3)) + w4 * rdot(d4, y4);
+    const float y1 = cget(A, i1, k), y2 = cget(A, i2, k), y3 = cget(A, i3, k), y4 = cget(A, i4, k);
+    const float s = ((w1 * quad_dot(d1, y1) + w2 * quad_dot(d2, y2)) + w3 * quad_dot(d3, y3)) + w4 * quad_dot(d4, y4);
     const float mubar = -s;
     const float cbar = (mubar / denom) * (six < 0.0f ? -1.0f : 1.0f);
     const float dbar_den = 2.0f * (-mubar * mu / denom);
-    const R3<float> e1 = (-mu * w1) * y1 + (dbar_den * w1) * d1, e2 = (-mu * w2) * y2 + (dbar_den * w2) * d2;
-    const R3<float> e3 = (-mu * w3) * y3 + (dbar_den * w3) * d3, e4 = (-mu * w4) * y4 + (dbar_den * w4) * d4;
-    R3<float> b1 = y1 + cbar * d1, b2 = y2 + cbar * d2, b3 = y3 + cbar * d3, b4 = y4 + cbar * d4;
+    const float e1 = (-mu * w1) * y1 + (dbar_den * w1) * d1, e2 = (-mu * w2) * y2 + (dbar_den * w2) * d2;
+    const float e3 = (-mu * w3) * y3 + (dbar_den * w3) * d3, e4 = (-mu * w4) * y4 + (dbar_den * w4) * d4;
+    float b1 = y1 + cbar * d1, b2 = y2 + cbar * d2, b3 = y3 + cbar * d3, b4 = y4 + cbar * d4;
     // d1 = (x4 - x2) x (x3 - x2)
-    R3<float> g = rcross(x2x3, e1), h = rcross(e1, x2x4);
+    float g = quad_cross(x2x3, e1), h = quad_cross(e1, x2x4);
     b4 = b4 + g; b3 = b3 + h; b2 = b2 - g - h;
     // d2 = (x3 - x1) x (x4 - x1)
-    g = rcross(x1x4, e2); h = rcross(e2, x1x3);
+    g = quad_cross(x1x4, e2); h = quad_cross(e2, x1x3);
     b3 = b3 + g; b4 = b4 + h; b1 = b1 - g - h;
     // d3 = (x4 - x1) x (x2 - x1)
-    g = rcross(x1x2, e3); h = rcross(e3, x1x4);
+    g = quad_cross(x1x2, e3); h = quad_cross(e3, x1x4);
     b4 = b4 + g; b2 = b2 + h; b1 = b1 - g - h;
     // d4 = (x2 - x1) x (x3 - x1)
-    g = rcross(x1x3, e4); h = rcross(e4, x1x2);
+    g = quad_cross(x1x3, e4); h = quad_cross(e4, x1x2);
     b2 = b2 + g; b3 = b3 + h; b1 = b1 - g - h;
-    A[i1] = make_float4(b1.x, b1.y, b1.z, a1.w);
-    A[i2] = make_float4(b2.x, b2.y, b2.z, a2.w);
-    A[i3] = make_float4(b3.x, b3.y, b3.z, a3.w);
-    A[i4] = make_float4(b4.x, b4.y, b4.z, a4.w);
+    if (!(denom < 1.0e-12f))
+    {
+        cset(A, i1, k, b1);
+        cset(A, i2, k, b2);
+        cset(A, i3, k, b3);
+        cset(A, i4, k, b4);
+    }
 }
 
-// Adjoint of edge_project from its pre-projection positions q0, q1.
-__device__ __forceinline__ void edge_adjoint(float4 *A, uint32_t i0, uint32_t i1, float4 q0, float4 q1, float rest,
-                                             float compliance, float inv_dt_sq, float &alpha_bar)
+// Adjoint of an edge from delta and length before its projection (formulas above), component k of
+// every vector per lane.  Returns what the edge adds to its compliance's adjoint.  Over hundreds of
+// sub-steps the position adjoints amplify rounding, so each of their quotients is the correctly
+// rounded one; the three that the quad shares are one division, a lane each.
+__device__ __forceinline__ float edge_adjoint(float4 *A, uint32_t lane, uint32_t k, uint32_t i0, uint32_t i1, float delta, float length,
+                                              float rest, float compliance, float inv_dt_sq)
 {
-    const R3<float> x0 = r3(q0.x, q0.y, q0.z), x1 = r3(q1.x, q1.y, q1.z);
-    const float w0 = q0.w, w1 = q1.w;
-    const R3<float> delta = x1 - x0;
-    const float length = sqrtf(rdot(delta, delta));
+    const float w0 = wget(A, i0), w1 = wget(A, i1);
     const float s = (w0 + w1) + compliance * inv_dt_sq;
     const float denom = length * s;
-    if (denom < 1.0e-12f)
-        return;
+    const bool acts = !(denom < 1.0e-12f);
     const float c = length - rest;
-    const R3<float> correction = (delta * c) / denom;
-    const float4 a0 = A[i0], a1 = A[i1];
-    const R3<float> ab0 = r3(a0.x, a0.y, a0.z), ab1 = r3(a1.x, a1.y, a1.z);
-    const R3<float> cbar = w0 * ab0 - w1 * ab1;
-    const R3<float> n = delta / length;
-    const R3<float> dbar = ((c / length) * cbar + ((rest / length) * rdot(n, cbar)) * n) / s;
-    A[i0] = make_float4(ab0.x - dbar.x, ab0.y - dbar.y, ab0.z - dbar.z, a0.w);
-    A[i1] = make_float4(ab1.x + dbar.x, ab1.y + dbar.y, ab1.z + dbar.z, a1.w);
-    alpha_bar += rdot(cbar, correction) * (-inv_dt_sq / s);
+    const float a0 = cget(A, i0, k), a1 = cget(A, i1, k);
+    const float cbar = w0 * a0 - w1 * a1;
+    const uint32_t l = lane & 3u;
+    const float q = (l == 0u ? c : l == 1u ? rest : 1.0f) / (l < 2u ? length : s);
+    const float c_length = quad_perm<kQuadX>(q), rest_length = quad_perm<kQuadY>(q), inv_s = quad_perm<kQuadZ>(q);
+    const float n = delta / length;
+    const float nc = quad_dot(n, cbar);
+    const float dbar = (c_length * cbar + (rest_length * nc) * n) / s;
+    if (acts)
+    {
+        cset(A, i0, k, a0 - dbar);
+        cset(A, i1, k, a1 + dbar);
+    }
+    // correction = n c / s, alphabar += (cbar . correction) (-1 / (h^2 s))
+    return acts ? (nc * c) * inv_s * (-inv_dt_sq * inv_s) : 0.0f;
 }
 
 template <class T> __device__ __forceinline__ R4<T> *state_vel(const RolloutDev &R);
@@ -396,12 +403,12 @@ template <> __device__ __forceinline__ R4<double> *state_prev<double>(const Roll
 // and the velocities V, with the operation order of the update kernel: GetVolumeTimesSix
 // (:107-118) summed in face order by one lane from per-face terms (terms: num_faces + 2 slots),
 // then each vertex adds its faces' impulses w * c * (x2 - x1) x (x3 - x1) in face order.
-template <class T>
+template <int BLOCK, class T>
 __device__ __forceinline__ void pressure_apply(const RolloutBodyDev &B, const StepConstants<T> &K, const R4<T> *X, R4<T> *V,
                                                T *terms, uint32_t tid)
 {
     const uint32_t nf = B.num_faces, nv = B.nv;
-    for (uint32_t f = tid; f < nf; f += kRolloutBlock)
+    for (uint32_t f = tid; f < nf; f += BLOCK)
     {
         const uint32_t *t = B.faces + 3u * f;
         terms[f] = rdot(rcross(xyz3(X[t[0]]), xyz3(X[t[1]])), xyz3(X[t[2]]));
@@ -419,7 +426,7 @@ __device__ __forceinline__ void pressure_apply(const RolloutBodyDev &B, const St
     if (six_volume > (T)0)
     {
         const T coefficient = (T)B.pressure * K.dt_sub / six_volume;
-        for (uint32_t i = tid; i < nv; i += kRolloutBlock)
+        for (uint32_t i = tid; i < nv; i += BLOCK)
         {
             const uint32_t fb = B.vf_begin[i], fe = B.vf_begin[i + 1];
             if (fb == fe)
@@ -452,12 +459,13 @@ __device__ __forceinline__ void atomic_add3(float4 *A, uint32_t i, const R3<floa
 // x1, x2, x3 through n_f = a x b: abar = b x nbar, bbar = nbar x a), Sbar = -cbar c / S (into
 // x1, x2, x3 through S: x2 x x3, x3 x x1, x1 x x2).  A (LDS) holds the position adjoints; faces
 // sharing a vertex add to it atomically.
+template <int BLOCK>
 __device__ __forceinline__ void pressure_adjoint(const RolloutBodyDev &B, float h, float4 *A, const float4 *vbar, const float4 *X0,
                                                  float *terms, uint32_t tid)
 {
     const uint32_t nf = B.num_faces;
     auto x_of = [&](uint32_t i) { const float4 q = X0[i]; return r3(q.x, q.y, q.z); };
-    for (uint32_t f = tid; f < nf; f += kRolloutBlock)
+    for (uint32_t f = tid; f < nf; f += BLOCK)
     {
         const uint32_t *t = B.faces + 3u * f;
         terms[f] = rdot(rcross(x_of(t[0]), x_of(t[1])), x_of(t[2]));
@@ -478,7 +486,7 @@ __device__ __forceinline__ void pressure_adjoint(const RolloutBodyDev &B, float 
     {
         const float c = B.pressure * h / S;
         float cb = 0.0f;
-        for (uint32_t f = tid; f < nf; f += kRolloutBlock)
+        for (uint32_t f = tid; f < nf; f += BLOCK)
         {
             const uint32_t *t = B.faces + 3u * f;
             const R3<float> x1 = x_of(t[0]), a = x_of(t[1]) - x1, b = x_of(t[2]) - x1;
@@ -497,7 +505,7 @@ __device__ __forceinline__ void pressure_adjoint(const RolloutBodyDev &B, float 
         atomicAdd(&terms[nf + 1], cb);
         __syncthreads();
         const float Sb = -terms[nf + 1] * c / S;
-        for (uint32_t f = tid; f < nf; f += kRolloutBlock)
+        for (uint32_t f = tid; f < nf; f += BLOCK)
         {
             const uint32_t *t = B.faces + 3u * f;
             const R3<float> x1 = x_of(t[0]), x2 = x_of(t[1]), x3 = x_of(t[2]);
@@ -512,15 +520,14 @@ __device__ __forceinline__ void pressure_adjoint(const RolloutBodyDev &B, float 
 // Pressure scratch after the LDS positions (and edge adjoints): num_faces + 2 slots of T
 template <class T> __device__ __forceinline__ T *pressure_terms(unsigned char *lds, uint32_t offset) { return reinterpret_cast<T *>(lds + offset); }
 
-// One sub-step of the forward pass on the LDS positions X; V / P are the
-// body's velocity / previous-position arrays.  The compliance of record r is
-// comp(r).
-template <class T, class Comp>
+// One sub-step of the forward pass on the LDS positions X; V / P are the body's velocity /
+// previous-position arrays.  project(): the constraint levels, ending in a workgroup barrier.
+template <int BLOCK, class T, class Project>
 __device__ __forceinline__ void forward_substep(const RolloutBodyDev &B, const StepConstants<T> &K, R4<T> *X, R4<T> *V, R4<T> *P,
-                                                bool last, uint32_t tid, Comp comp)
+                                                bool last, uint32_t tid, Project project)
 {
     const uint32_t nv = B.nv;
-    for (uint32_t i = tid; i < nv; i += kRolloutBlock)
+    for (uint32_t i = tid; i < nv; i += BLOCK)
     {
         const R4<T> p = X[i];
         const R3<T> v = K.integrate_velocity(xyz3(V[i]), p.w);
@@ -530,30 +537,8 @@ __device__ __forceinline__ void forward_substep(const RolloutBodyDev &B, const S
         V[i] = r4(v, (T)0);
     }
     __syncthreads();
-    if (B.edges_only)
-        run_program_global<kRolloutBlock, false>(B.recs, B.lvl, B.nlev, tid, [&](const uint4 &q, uint32_t) {
-            if (q.x != kNopRecord)
-                edge_project<T>(X, q.x & 0x3fffu, q.x >> 16, (T)__uint_as_float(q.z), comp(q), K.inv_dt_sq);
-        });
-    else
-        run_program_global<kRolloutBlock, false>(B.recs, B.lvl, B.nlev, tid, [&](const uint4 &q, uint32_t) {
-            if (q.x == kNopRecord)
-                return;
-            if (is_lra_record(q))
-                lra_project<T>(X, q.x & 0x3fffu, q.x >> 16, (T)__uint_as_float(q.z));
-            else if (is_bend_record(q))
-            {
-                if (!is_second_half(q))
-                    bend_project<T>(X, q.x & 0x3fffu, q.x >> 16, q.y & 0x7fffu, q.y >> 16, __uint_as_float(q.z),
-                                    __uint_as_float(q.w), K.inv_dt_sq);
-            }
-            else if (is_volume_record(q))
-                volume_project<T>(X, q.x & 0x3fffu, q.x >> 16, q.y & 0x7fffu, q.y >> 16, (T)__uint_as_float(q.z),
-                                  (T)__uint_as_float(q.w), K.inv_dt_sq);
-            else
-                edge_project<T>(X, q.x & 0x3fffu, q.x >> 16, (T)__uint_as_float(q.z), comp(q), K.inv_dt_sq);
-        });
-    for (uint32_t i = tid; i < nv; i += kRolloutBlock)
+    project();
+    for (uint32_t i = tid; i < nv; i += BLOCK)
     {
         const R4<T> p = X[i];
         R3<T> v = xyz3(V[i]);
@@ -570,12 +555,147 @@ __device__ __forceinline__ void forward_substep(const RolloutBodyDev &B, const S
     __syncthreads();
 }
 
-// Forward pass.  The float pass first writes each record's compliance into
-// the record (.w), where the backward pass reads it, and stores the (x, v)
-// checkpoints; the double pass reads the compliance array directly.
-template <class T>
-__global__ __launch_bounds__(kRolloutBlock) void rollout_forward_kernel(RolloutDev R, const T *__restrict__ compliance,
-                                                                      const T *__restrict__ velocity, T *__restrict__ positions)
+// The constraint levels in double, on the level program; comp(r): the compliance of record r
+template <class Comp>
+__device__ __forceinline__ void project_levels(const RolloutBodyDev &B, const StepConstants<double> &K, R4<double> *X, uint32_t tid, Comp comp)
+{
+    using T = double;
+    if (B.edges_only)
+        run_program_global<kRolloutDoubleBlock, false>(B.recs, B.lvl, B.nlev, tid, [&](const uint4 &q, uint32_t) {
+            if (q.x != kNopRecord)
+                edge_project<T>(X, q.x & 0x3fffu, q.x >> 16, (T)__uint_as_float(q.z), comp(q), K.inv_dt_sq);
+        });
+    else
+        run_program_global<kRolloutDoubleBlock, false>(B.recs, B.lvl, B.nlev, tid, [&](const uint4 &q, uint32_t) {
+            if (q.x == kNopRecord)
+                return;
+            if (is_lra_record(q))
+                lra_project<T>(X, q.x & 0x3fffu, q.x >> 16, (T)__uint_as_float(q.z));
+            else if (is_bend_record(q))
+            {
+                if (!is_second_half(q))
+                    bend_project<T>(X, q.x & 0x3fffu, q.x >> 16, q.y & 0x7fffu, q.y >> 16, __uint_as_float(q.z),
+                                    __uint_as_float(q.w), K.inv_dt_sq);
+            }
+            else if (is_volume_record(q))
+                volume_project<T>(X, q.x & 0x3fffu, q.x >> 16, q.y & 0x7fffu, q.y >> 16, (T)__uint_as_float(q.z),
+                                  (T)__uint_as_float(q.w), K.inv_dt_sq);
+            else
+                edge_project<T>(X, q.x & 0x3fffu, q.x >> 16, (T)__uint_as_float(q.z), comp(q), K.inv_dt_sq);
+        });
+}
+
+// The constraint levels in float, as the task program (the projections of the update kernels).
+// TAPE: what each record's adjoint needs goes to `tape`, in record order.
+template <bool TAPE, bool BENDS>
+__device__ __forceinline__ void project_tasks(const RolloutBodyDev &B, float4 *X, float inv_dt_sq, uint32_t tid, float4 *tape)
+{
+    const uint32_t lane = tid & (kWave - 1u), quad = lane >> 2, c = (lane & 3u) < 2u ? (lane & 3u) : 2u;
+    const uint32_t stride = B.tape_stride;
+    TaskStream<> tasks;
+    tasks.begin(B.task_recs, B.task_desc, B.task_heads + (tid >> 6), lane);
+    tasks.run(lane, [&](uint32_t d, const uint4 &r, NoAux::Value, uint32_t first) {
+        const uint32_t n = d & 127u, kind = (d >> 7) & 7u;
+        const uint32_t i0 = r.x & 0x3fffu, i1 = r.x >> 16, i2 = r.y & 0x3fffu, i3 = r.y >> 16;
+        const float p0 = __uint_as_float(r.z), p1 = __uint_as_float(r.w);
+        if (kind == kTaskEdgeQuad)
+        {
+            if (quad < n)
+            {
+                float delta, length;
+                project_edge_quad(X, c, i0, i1, p0, p1, inv_dt_sq, delta, length);
+                if (TAPE)
+                    reinterpret_cast<float *>(tape + (size_t)stride * (first + quad))[lane & 3u] = (lane & 3u) == 3u ? length : delta;
+            }
+        }
+        else if (kind == kTaskVolumeQuad || (BENDS && kind == kTaskBendQuad))
+        {
+            if (quad < n)
+            {
+                if (TAPE && (lane & 3u) < 3u)
+                    tape[(size_t)stride * (first + quad) + c] = make_float4(cget(X, i0, c), cget(X, i1, c), cget(X, i2, c), cget(X, i3, c));
+                if (BENDS && kind == kTaskBendQuad)
+                    project_bend_quad(X, c, i0, i1, i2, i3, p0, p1, inv_dt_sq);
+                else
+                    project_volume_quad(X, c, i0, i1, i2, i3, p0, p1, inv_dt_sq);
+            }
+        }
+        else if (lane < n && i0 != i1)
+        {
+            if (TAPE)
+            {
+                const V3 delta = xyz(X[i1]) - xyz(X[i0]);
+                tape[(size_t)stride * (first + lane)] = f4(delta, len_sq(delta));
+            }
+            project_lra(X, i0, i1, p0);
+        }
+    });
+}
+
+// Tape entries the reverse run loads ahead: {delta, length} or, for a volume, the lane's component
+// of the four positions (a bend loads its three entries itself)
+struct TapeAux
+{
+    using Value = RecordVec;
+    const float4 *tape;
+    uint32_t stride;
+    __device__ __forceinline__ Value load(uint32_t record, uint32_t d, uint32_t lane) const
+    {
+        const uint32_t c = ((d >> 7) & 7u) == kTaskVolumeQuad ? ((lane & 3u) < 2u ? (lane & 3u) : 2u) : 0u;
+        return load_record(reinterpret_cast<const uint4 *>(tape + (size_t)stride * record), c);
+    }
+};
+
+// The adjoint of the constraint levels: the task program backwards on the position adjoints A
+// (xyz; w: inverse mass), ending in a workgroup barrier.
+template <bool BENDS>
+__device__ __forceinline__ void reverse_tasks(const RolloutBodyDev &B, float4 *A, float *alpha_bar, float inv_dt_sq, uint32_t tid,
+                                              const float4 *tape)
+{
+    const uint32_t lane = tid & (kWave - 1u), quad = lane >> 2, c = (lane & 3u) < 2u ? (lane & 3u) : 2u;
+    const TapeAux aux{ tape, B.tape_stride };
+    TaskStream<true, TapeAux> tasks;
+    tasks.begin(B.task_recs, B.task_desc, B.task_heads + (tid >> 6), lane, aux);
+    tasks.run(lane, [&](uint32_t d, const uint4 &r, const RecordVec &tv, uint32_t first) {
+        const uint32_t n = d & 127u, kind = (d >> 7) & 7u;
+        const uint32_t i0 = r.x & 0x3fffu, i1 = r.x >> 16, i2 = r.y & 0x3fffu, i3 = r.y >> 16;
+        const float p0 = __uint_as_float(r.z), p1 = __uint_as_float(r.w);
+        const float4 t = make_float4(__uint_as_float(tv.x), __uint_as_float(tv.y), __uint_as_float(tv.z), __uint_as_float(tv.w));
+        if (kind == kTaskEdgeQuad)
+        {
+            if (quad < n)
+            {
+                const float delta = c == 0 ? t.x : c == 1 ? t.y : t.z;
+                const float alpha = edge_adjoint(A, lane, c, i0, i1, delta, t.w, p0, p1, inv_dt_sq);
+                if ((lane & 3u) == 0u)
+                    alpha_bar[r.y] += alpha;
+            }
+        }
+        else if (kind == kTaskVolumeQuad)
+        {
+            if (quad < n)
+                volume_adjoint(A, c, i0, i1, i2, i3, t, p0, p1, inv_dt_sq);
+        }
+        else if (BENDS && kind == kTaskBendQuad)
+        {
+            if (quad < n)
+            {
+                const float4 *q = tape + (size_t)B.tape_stride * (first + quad);
+                bend_adjoint(A, lane, i0, i1, i2, i3, q[0], q[1], q[2], p0, p1, inv_dt_sq);
+            }
+        }
+        else if (lane < n && i0 != i1)
+            lra_adjoint(A, i0, i1, t, p0);
+    }, aux);
+    __syncthreads();
+}
+
+// Forward pass.  The float pass first writes each edge's compliance into its task record (.w),
+// where the backward pass reads it, and stores the (x, v) checkpoints; the double pass reads the
+// compliance array directly.
+template <class T, int BLOCK>
+__global__ __launch_bounds__(BLOCK) void rollout_forward_kernel(RolloutDev R, const T *__restrict__ compliance,
+                                                                const T *__restrict__ velocity, T *__restrict__ positions)
 {
     extern __shared__ __align__(16) unsigned char lds_raw[];
     R4<T> *X = reinterpret_cast<R4<T> *>(lds_raw);
@@ -587,38 +707,28 @@ __global__ __launch_bounds__(kRolloutBlock) void rollout_forward_kernel(RolloutD
     R4<T> *P = state_prev<T>(R) + B.voff;
     constexpr bool kFloat = sizeof(T) == 4;
     if (kFloat)
-    {
-        uint4 *recs = const_cast<uint4 *>(B.recs);
-        for (uint32_t r = tid; r < B.num_records; r += kRolloutBlock)
+        for (uint32_t r = tid; r < B.num_task_records; r += BLOCK)
         {
-            uint4 q = recs[r];
-            if (q.x != kNopRecord && !is_lra_record(q) && !is_volume_record(q) && !is_bend_record(q))
-            {
-                q.w = __float_as_uint((float)compliance[B.eoff + q.y]);
-                recs[r] = q;
-            }
+            const uint4 q = B.task_recs[r];
+            if (((q.x >> 14) & 3u) == kTypeEdge)
+                B.task_recs[r].w = __float_as_uint((float)compliance[B.eoff + q.y]);
         }
-    }
-    for (uint32_t i = tid; i < nv; i += kRolloutBlock)
+    for (uint32_t i = tid; i < nv; i += BLOCK)
     {
         X[i] = to_r4<T>(B.x0[i]);
         const uint32_t g = 3u * (B.voff + i);
         R4<T> v; v.x = velocity[g]; v.y = velocity[g + 1]; v.z = velocity[g + 2]; v.w = (T)0;
         V[i] = v;
     }
-    __syncthreads();
+    // other wavefronts read the compliances this one wrote
+    sync_global();
     const StepConstants<T> K(R, nv);
-    auto comp = [&](const uint4 &q) -> T {
-        if (kFloat)
-            return (T)__uint_as_float(q.w);
-        return compliance[B.eoff + q.y];
-    };
     for (uint32_t frame = 0; frame < R.frames; ++frame)
     {
         if (kFloat && frame % R.interval == 0)
         {
             const size_t base = (size_t)(frame / R.interval) * R.total_nv + B.voff;
-            for (uint32_t i = tid; i < nv; i += kRolloutBlock)
+            for (uint32_t i = tid; i < nv; i += BLOCK)
             {
                 const R4<T> p = X[i], v = V[i];
                 R.ckpt_x[base + i] = make_float4((float)p.x, (float)p.y, (float)p.z, (float)p.w);
@@ -628,11 +738,16 @@ __global__ __launch_bounds__(kRolloutBlock) void rollout_forward_kernel(RolloutD
         for (uint32_t it = 0; it < R.iterations; ++it)
         {
             if (B.num_faces > 0)
-                pressure_apply<T>(B, K, X, V, terms, tid);
-            forward_substep<T>(B, K, X, V, P, it + 1 == R.iterations, tid, comp);
+                pressure_apply<BLOCK, T>(B, K, X, V, terms, tid);
+            forward_substep<BLOCK, T>(B, K, X, V, P, it + 1 == R.iterations, tid, [&]() {
+                if constexpr (kFloat)
+                    project_tasks<false, true>(B, reinterpret_cast<float4 *>(X), K.inv_dt_sq, tid, nullptr);
+                else
+                    project_levels(B, K, X, tid, [&](const uint4 &q) -> double { return compliance[B.eoff + q.y]; });
+            });
         }
     }
-    for (uint32_t i = tid; i < nv; i += kRolloutBlock)
+    for (uint32_t i = tid; i < nv; i += BLOCK)
     {
         const uint32_t g = 3u * (B.voff + i);
         const R4<T> p = X[i];
@@ -640,10 +755,15 @@ __global__ __launch_bounds__(kRolloutBlock) void rollout_forward_kernel(RolloutD
     }
 }
 
-// Adjoint of the last float forward pass.
-__global__ __launch_bounds__(kRolloutBlock) void rollout_backward_kernel(RolloutDev R, const float *__restrict__ grad_positions,
-                                                                       float *__restrict__ grad_compliance,
-                                                                       float *__restrict__ grad_velocity)
+// Adjoint of the last float forward pass.  Per segment, last first: recompute it from its
+// checkpoint keeping every sub-step's start state and, when it fits (R.tape_subs), every
+// sub-step's tape; then reverse it sub-step by sub-step.  A tape of one sub-step is filled by
+// running the sub-step again before its adjoint.  Measured on 64 cloths of 64 x 64 (60 frames x 5
+// iterations), forward and adjoint: 229 -> 114 ms; before, every sub-step ran a second forward
+// sweep for its tape, whose loads stood exposed in every reverse level.
+template <int BLOCK, bool BENDS>
+__global__ __launch_bounds__(BLOCK) void rollout_backward_kernel(RolloutDev R, const float *__restrict__ grad_positions,
+                                                                 float *__restrict__ grad_compliance, float *__restrict__ grad_velocity)
 {
     extern __shared__ __align__(16) unsigned char lds_raw[];
     const uint32_t tid = threadIdx.x;
@@ -657,11 +777,10 @@ __global__ __launch_bounds__(kRolloutBlock) void rollout_backward_kernel(Rollout
     R4<float> *V = state_vel<float>(R) + B.voff;
     R4<float> *P = state_prev<float>(R) + B.voff;
     float4 *adj_x = R.adj_x + B.voff, *adj_v = R.adj_v + B.voff;
-    float4 *tape = R.rec_tape + 4u * (size_t)B.rbase;
 
-    for (uint32_t e = tid; e < ne; e += kRolloutBlock)
+    for (uint32_t e = tid; e < ne; e += BLOCK)
         alpha_bar[e] = 0.0f;
-    for (uint32_t i = tid; i < nv; i += kRolloutBlock)
+    for (uint32_t i = tid; i < nv; i += BLOCK)
     {
         const uint32_t g = 3u * (B.voff + i);
         adj_x[i] = make_float4(grad_positions[g], grad_positions[g + 1], grad_positions[g + 2], 0.0f);
@@ -669,7 +788,6 @@ __global__ __launch_bounds__(kRolloutBlock) void rollout_backward_kernel(Rollout
     }
     const StepConstants<float> K(R, nv);
     const float h = K.dt_sub;
-    auto comp = [](const uint4 &q) -> float { return __uint_as_float(q.w); };
     const uint32_t I = R.iterations;
     const uint32_t num_ckpt = (R.frames + R.interval - 1) / R.interval;
     __syncthreads();
@@ -679,9 +797,11 @@ __global__ __launch_bounds__(kRolloutBlock) void rollout_backward_kernel(Rollout
         const uint32_t f0 = seg * R.interval;
         const uint32_t f1 = f0 + R.interval < R.frames ? f0 + R.interval : R.frames;
         const uint32_t nsub = (f1 - f0) * I;
-        // recompute the segment from its checkpoint, keeping every sub-step's start state
+        const bool whole = nsub <= R.tape_subs;
+        float4 *tape0 = R.tape + B.tape_offset;
+        // recompute the segment from its checkpoint
         const size_t cbase = (size_t)seg * R.total_nv + B.voff;
-        for (uint32_t i = tid; i < nv; i += kRolloutBlock)
+        for (uint32_t i = tid; i < nv; i += BLOCK)
         {
             const float4 p = R.ckpt_x[cbase + i], v = R.ckpt_v[cbase + i];
             X[i] = to_r4<float>(p);
@@ -693,126 +813,70 @@ __global__ __launch_bounds__(kRolloutBlock) void rollout_backward_kernel(Rollout
             const size_t sbase = (size_t)s * R.total_nv + B.voff;
             // the tape keeps the velocity after the pressure step
             if (has_pressure)
-                pressure_apply<float>(B, K, X, V, terms, tid);
-            for (uint32_t i = tid; i < nv; i += kRolloutBlock)
+                pressure_apply<BLOCK, float>(B, K, X, V, terms, tid);
+            for (uint32_t i = tid; i < nv; i += BLOCK)
             {
                 R.seg_x[sbase + i] = A[i];
                 R.seg_v[sbase + i] = to_f4(V[i]);
             }
-            forward_substep<float>(B, K, X, V, P, s % I == I - 1, tid, comp);
+            forward_substep<BLOCK, float>(B, K, X, V, P, s % I == I - 1, tid, [&]() {
+                if (whole)
+                    project_tasks<true, BENDS>(B, A, K.inv_dt_sq, tid, tape0 + (size_t)s * R.tape_size);
+                else
+                    project_tasks<false, BENDS>(B, A, K.inv_dt_sq, tid, nullptr);
+            });
         }
+        for (uint32_t i = tid; i < nv; i += BLOCK)
+            R.seg_x[(size_t)nsub * R.total_nv + B.voff + i] = A[i];
         // reverse the segment sub-step by sub-step
         for (uint32_t s = nsub; s-- > 0;)
         {
             const size_t sbase = (size_t)s * R.total_nv + B.voff;
             const bool last = s % I == I - 1;
-            // re-run the sub-step, recording every edge's pre-projection positions
-            for (uint32_t i = tid; i < nv; i += kRolloutBlock)
+            if (!whole)
             {
-                const float4 p = R.seg_x[sbase + i], v0 = R.seg_v[sbase + i];
-                const R3<float> v1 = K.integrate_velocity(r3(v0.x, v0.y, v0.z), p.w);
-                X[i] = r4(r3(p.x, p.y, p.z) + v1 * h, p.w);
+                // run the sub-step again, recording its tape
+                __syncthreads();
+                for (uint32_t i = tid; i < nv; i += BLOCK)
+                {
+                    const float4 p = R.seg_x[sbase + i], v0 = R.seg_v[sbase + i];
+                    const R3<float> v1 = K.integrate_velocity(r3(v0.x, v0.y, v0.z), p.w);
+                    X[i] = r4(r3(p.x, p.y, p.z) + v1 * h, p.w);
+                }
+                __syncthreads();
+                project_tasks<true, BENDS>(B, A, K.inv_dt_sq, tid, tape0);
             }
-            __syncthreads();
-            if (B.edges_only)
-                run_program_global<kRolloutBlock, false>(B.recs, B.lvl, B.nlev, tid, [&](const uint4 &q, uint32_t r) {
-                    if (q.x == kNopRecord)
-                        return;
-                    const uint32_t i0 = q.x & 0x3fffu, i1 = q.x >> 16;
-                    tape[4u * r] = A[i0];
-                    tape[4u * r + 1u] = A[i1];
-                    edge_project<float>(X, i0, i1, __uint_as_float(q.z), __uint_as_float(q.w), K.inv_dt_sq);
-                });
-            else
-                run_program_global<kRolloutBlock, false>(B.recs, B.lvl, B.nlev, tid, [&](const uint4 &q, uint32_t r) {
-                    if (q.x == kNopRecord)
-                        return;
-                    const uint32_t i0 = q.x & 0x3fffu, i1 = q.x >> 16;
-                    tape[4u * r] = A[i0];
-                    tape[4u * r + 1u] = A[i1];
-                    if (is_volume_record(q))
-                    {
-                        const uint32_t i2 = q.y & 0x7fffu, i3 = q.y >> 16;
-                        tape[4u * r + 2u] = A[i2];
-                        tape[4u * r + 3u] = A[i3];
-                        volume_project<float>(X, i0, i1, i2, i3, __uint_as_float(q.z), __uint_as_float(q.w), K.inv_dt_sq);
-                    }
-                    else if (is_bend_record(q))
-                    {
-                        if (!is_second_half(q))
-                        {
-                            const uint32_t i2 = q.y & 0x7fffu, i3 = q.y >> 16;
-                            tape[4u * r + 2u] = A[i2];
-                            tape[4u * r + 3u] = A[i3];
-                            bend_project<float>(X, i0, i1, i2, i3, __uint_as_float(q.z), __uint_as_float(q.w), K.inv_dt_sq);
-                        }
-                    }
-                    else if (is_lra_record(q))
-                        lra_project<float>(X, i0, i1, __uint_as_float(q.z));
-                    else
-                        edge_project<float>(X, i0, i1, __uint_as_float(q.z), __uint_as_float(q.w), K.inv_dt_sq);
-                });
+            // the tape was written by other lanes
+            sync_global();
             // adjoint of the velocity update (and of the clamp after the last iteration)
-            for (uint32_t i = tid; i < nv; i += kRolloutBlock)
+            for (uint32_t i = tid; i < nv; i += BLOCK)
             {
-                const float4 p = R.seg_x[sbase + i], v0 = R.seg_v[sbase + i];
-                const float w = p.w;
-                const R3<float> x0 = r3(p.x, p.y, p.z);
-                const R3<float> v1 = K.integrate_velocity(r3(v0.x, v0.y, v0.z), w);
-                const R3<float> y = xyz3(X[i]);
-                const R3<float> v2 = w > 0.0f ? (y - x0) / h : v1;
+                const float w = B.x0[i].w;
                 const float4 vbf = adj_v[i], xbf = adj_x[i];
                 R3<float> vb = r3(vbf.x, vbf.y, vbf.z);
                 if (last)
                 {
+                    const float4 p = R.seg_x[sbase + i], v0 = R.seg_v[sbase + i], y = R.seg_x[sbase + R.total_nv + i];
+                    const R3<float> v1 = K.integrate_velocity(r3(v0.x, v0.y, v0.z), w);
+                    const R3<float> v2 = w > 0.0f ? (r3(y.x, y.y, y.z) - r3(p.x, p.y, p.z)) / h : v1;
                     const float v_sq = rdot(v2, v2);
                     if (v_sq > K.max_lin_sq)
                     {
                         const float l = sqrtf(v_sq);
                         const R3<float> n = v2 / l;
                         vb = (sqrtf(K.max_lin_sq) / l) * (vb - rdot(n, vb) * n);
+                        adj_v[i] = make_float4(vb.x, vb.y, vb.z, 0.0f);
                     }
                 }
-                adj_v[i] = make_float4(vb.x, vb.y, vb.z, 0.0f);
                 R3<float> yb = r3(xbf.x, xbf.y, xbf.z);
                 if (w > 0.0f)
                     yb = yb + vb / h;
                 A[i] = make_float4(yb.x, yb.y, yb.z, w);
             }
             __syncthreads();
-            if (B.edges_only)
-                run_program_global<kRolloutBlock, true>(B.recs, B.lvl, B.nlev, tid, [&](const uint4 &q, uint32_t r) {
-                    if (q.x != kNopRecord)
-                        edge_adjoint(A, q.x & 0x3fffu, q.x >> 16, tape[4u * r], tape[4u * r + 1u], __uint_as_float(q.z),
-                                     __uint_as_float(q.w), K.inv_dt_sq, alpha_bar[q.y]);
-                });
-            else
-                run_program_global<kRolloutBlock, true>(B.recs, B.lvl, B.nlev, tid, [&](const uint4 &q, uint32_t r) {
-                    if (q.x == kNopRecord)
-                        return;
-                    if (is_lra_record(q))
-                    {
-                        lra_adjoint(A, q.x & 0x3fffu, q.x >> 16, tape[4u * r], tape[4u * r + 1u], __uint_as_float(q.z));
-                        return;
-                    }
-                    if (is_bend_record(q))
-                    {
-                        if (!is_second_half(q))
-                            bend_adjoint(A, q.x & 0x3fffu, q.x >> 16, q.y & 0x7fffu, q.y >> 16, tape + 4u * r, __uint_as_float(q.z),
-                                         __uint_as_float(q.w), K.inv_dt_sq);
-                        return;
-                    }
-                    if (is_volume_record(q))
-                    {
-                        volume_adjoint(A, q.x & 0x3fffu, q.x >> 16, q.y & 0x7fffu, q.y >> 16, tape + 4u * r, __uint_as_float(q.z),
-                                       __uint_as_float(q.w), K.inv_dt_sq);
-                        return;
-                    }
-                    edge_adjoint(A, q.x & 0x3fffu, q.x >> 16, tape[4u * r], tape[4u * r + 1u], __uint_as_float(q.z),
-                                 __uint_as_float(q.w), K.inv_dt_sq, alpha_bar[q.y]);
-                });
+            reverse_tasks<BENDS>(B, A, alpha_bar, K.inv_dt_sq, tid, tape0 + (whole ? (size_t)s * R.tape_size : 0));
             // adjoint of prev = x0, y0 = x0 + v1 h and the integration of v
-            for (uint32_t i = tid; i < nv; i += kRolloutBlock)
+            for (uint32_t i = tid; i < nv; i += BLOCK)
             {
                 const float4 yb4 = A[i], vbf = adj_v[i];
                 const float w = yb4.w;
@@ -829,28 +893,32 @@ __global__ __launch_bounds__(kRolloutBlock) void rollout_backward_kernel(Rollout
                     adj_x[i] = make_float4(x0b.x, x0b.y, x0b.z, 0.0f);
                 adj_v[i] = make_float4(v0b.x, v0b.y, v0b.z, 0.0f);
             }
-            __syncthreads();
             if (has_pressure)
             {
-                pressure_adjoint(B, h, A, adj_v, R.seg_x + sbase, terms, tid);
-                for (uint32_t i = tid; i < nv; i += kRolloutBlock)
+                // the adjoint reads the velocities' adjoints of other lanes
+                sync_global();
+                pressure_adjoint<BLOCK>(B, h, A, adj_v, R.seg_x + sbase, terms, tid);
+                for (uint32_t i = tid; i < nv; i += BLOCK)
                 {
                     const float4 a = A[i];
                     adj_x[i] = make_float4(a.x, a.y, a.z, 0.0f);
                 }
-                __syncthreads();
             }
         }
+        __syncthreads();
     }
-    for (uint32_t i = tid; i < nv; i += kRolloutBlock)
+    for (uint32_t i = tid; i < nv; i += BLOCK)
     {
         const uint32_t g = 3u * (B.voff + i);
         const float4 v = adj_v[i];
         grad_velocity[g] = v.x; grad_velocity[g + 1] = v.y; grad_velocity[g + 2] = v.z;
     }
-    for (uint32_t e = tid; e < ne; e += kRolloutBlock)
+    for (uint32_t e = tid; e < ne; e += BLOCK)
         grad_compliance[B.eoff + e] = alpha_bar[e];
 }
+
+// Wavefronts of the float passes' workgroups: the task programs are built for them
+uint32_t rollout_waves(bool bends) { return (uint32_t)(bends ? kRolloutBendBlock : kRolloutBlock) / kWave; }
 
 // nf: faces under pressure (0: none), which add num_faces + 2 scratch slots
 uint32_t rollout_forward_lds_bytes(uint32_t nv, uint32_t nf, bool f64)
@@ -868,15 +936,24 @@ static hipError_t allow_lds(K kernel)
     return hipFuncSetAttribute((const void *)kernel, hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024 - 1024);
 }
 
-hipError_t launch_rollout_forward_f32(const RolloutDev &R, const float *compliance, const float *velocity, float *positions,
-                                      uint32_t lds, hipStream_t stream)
+template <int BLOCK>
+static hipError_t launch_forward_block(const RolloutDev &R, const float *compliance, const float *velocity, float *positions,
+                                       uint32_t lds, hipStream_t stream)
 {
-    static hipError_t configured = allow_lds(rollout_forward_kernel<float>);
+    static hipError_t configured = allow_lds(rollout_forward_kernel<float, BLOCK>);
     if (configured != hipSuccess)
         return configured;
-    hipLaunchKernelGGL(rollout_forward_kernel<float>, dim3(R.num_bodies), dim3(kRolloutBlock), lds, stream, R, compliance,
+    hipLaunchKernelGGL((rollout_forward_kernel<float, BLOCK>), dim3(R.num_bodies), dim3(BLOCK), lds, stream, R, compliance,
                        velocity, positions);
     return hipGetLastError();
+}
+
+// bends: some body has dihedral bends (every body then runs in the smaller workgroups)
+hipError_t launch_rollout_forward_f32(const RolloutDev &R, bool bends, const float *compliance, const float *velocity, float *positions,
+                                      uint32_t lds, hipStream_t stream)
+{
+    return bends ? launch_forward_block<kRolloutBendBlock>(R, compliance, velocity, positions, lds, stream)
+                 : launch_forward_block<kRolloutBlock>(R, compliance, velocity, positions, lds, stream);
 }
 
 // ---------------------------------------------------------------- no-allocation forward
@@ -916,7 +993,7 @@ hipError_t rollout_scratch_setup(int device)
 
 // The float forward with R.vel / R.prev in this device's scratch array.  The caller has
 // checked R.total_nv against kNoAllocMaxVertices; allocates nothing.
-hipError_t launch_rollout_forward_f32_noalloc(int device, RolloutDev R, const float *compliance, const float *velocity,
+hipError_t launch_rollout_forward_f32_noalloc(int device, RolloutDev R, bool bends, const float *compliance, const float *velocity,
                                               float *positions, uint32_t lds, hipStream_t stream)
 {
     if (device < 0 || device >= kMaxScratchDevices || R.total_nv > kNoAllocMaxVertices)
@@ -930,29 +1007,37 @@ hipError_t launch_rollout_forward_f32_noalloc(int device, RolloutDev R, const fl
         return hipErrorNotInitialized;
     R.vel = base;
     R.prev = base + kNoAllocMaxVertices;
-    return launch_rollout_forward_f32(R, compliance, velocity, positions, lds, stream);
+    return launch_rollout_forward_f32(R, bends, compliance, velocity, positions, lds, stream);
 }
 
 hipError_t launch_rollout_forward_f64(const RolloutDev &R, const double *compliance, const double *velocity, double *positions,
                                       uint32_t lds, hipStream_t stream)
 {
-    static hipError_t configured = allow_lds(rollout_forward_kernel<double>);
+    static hipError_t configured = allow_lds(rollout_forward_kernel<double, kRolloutDoubleBlock>);
     if (configured != hipSuccess)
         return configured;
-    hipLaunchKernelGGL(rollout_forward_kernel<double>, dim3(R.num_bodies), dim3(kRolloutBlock), lds, stream, R, compliance,
+    hipLaunchKernelGGL((rollout_forward_kernel<double, kRolloutDoubleBlock>), dim3(R.num_bodies), dim3(kRolloutDoubleBlock), lds, stream, R, compliance,
                        velocity, positions);
     return hipGetLastError();
 }
 
-hipError_t launch_rollout_backward(const RolloutDev &R, const float *grad_positions, float *grad_compliance, float *grad_velocity,
-                                   uint32_t lds, hipStream_t stream)
+template <int BLOCK, bool BENDS>
+static hipError_t launch_backward_block(const RolloutDev &R, const float *grad_positions, float *grad_compliance, float *grad_velocity,
+                                        uint32_t lds, hipStream_t stream)
 {
-    static hipError_t configured = allow_lds(rollout_backward_kernel);
+    static hipError_t configured = allow_lds(rollout_backward_kernel<BLOCK, BENDS>);
     if (configured != hipSuccess)
         return configured;
-    hipLaunchKernelGGL(rollout_backward_kernel, dim3(R.num_bodies), dim3(kRolloutBlock), lds, stream, R, grad_positions,
+    hipLaunchKernelGGL((rollout_backward_kernel<BLOCK, BENDS>), dim3(R.num_bodies), dim3(BLOCK), lds, stream, R, grad_positions,
                        grad_compliance, grad_velocity);
     return hipGetLastError();
+}
+
+hipError_t launch_rollout_backward(const RolloutDev &R, bool bends, const float *grad_positions, float *grad_compliance, float *grad_velocity,
+                                   uint32_t lds, hipStream_t stream)
+{
+    return bends ? launch_backward_block<kRolloutBendBlock, true>(R, grad_positions, grad_compliance, grad_velocity, lds, stream)
+                 : launch_backward_block<kRolloutBlock, false>(R, grad_positions, grad_compliance, grad_velocity, lds, stream);
 }
 
 } // namespace xpbd

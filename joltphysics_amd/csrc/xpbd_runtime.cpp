@@ -39,15 +39,16 @@ hipError_t launch_skin(const float *joints, const SkinInvBindDev *inv_binds, uin
                        float4 *states, uint32_t nv, float4 *x, float4 *v, int32_t hard_skin_all, hipStream_t stream);
 uint32_t rollout_forward_lds_bytes(uint32_t nv, uint32_t nf, bool f64);
 uint32_t rollout_backward_lds_bytes(uint32_t nv, uint32_t ne, uint32_t nf);
-hipError_t launch_rollout_forward_f32(const RolloutDev &R, const float *compliance, const float *velocity, float *positions,
+uint32_t rollout_waves(bool bends);
+hipError_t launch_rollout_forward_f32(const RolloutDev &R, bool bends, const float *compliance, const float *velocity, float *positions,
                                       uint32_t lds, hipStream_t stream);
 hipError_t launch_rollout_forward_f64(const RolloutDev &R, const double *compliance, const double *velocity, double *positions,
                                       uint32_t lds, hipStream_t stream);
-hipError_t launch_rollout_backward(const RolloutDev &R, const float *grad_positions, float *grad_compliance, float *grad_velocity,
+hipError_t launch_rollout_backward(const RolloutDev &R, bool bends, const float *grad_positions, float *grad_compliance, float *grad_velocity,
                                    uint32_t lds, hipStream_t stream);
 hipError_t rollout_scratch_setup(int device);
 uint32_t rollout_noalloc_max_vertices();
-hipError_t launch_rollout_forward_f32_noalloc(int device, RolloutDev R, const float *compliance, const float *velocity,
+hipError_t launch_rollout_forward_f32_noalloc(int device, RolloutDev R, bool bends, const float *compliance, const float *velocity,
                                               float *positions, uint32_t lds, hipStream_t stream);
 } // namespace xpbd
 
@@ -487,8 +488,9 @@ struct GroupLevels
 struct TaskProgram
 {
     std::vector<uint4> recs;        // per wavefront, in task order; one record behind the last
-    std::vector<uint32_t> desc;     // per wavefront, kDescPad zero descriptors behind each list
-    std::vector<uint4> heads;       // per wavefront {first descriptor, tasks, first record, trailing barriers}
+    std::vector<uint32_t> desc;     // per wavefront, kDescPad zero descriptors before and behind each list
+    std::vector<uint4> heads;       // per wavefront {first descriptor, tasks, first record, trailing barriers}, then
+                                    // one with the end of the records
     double ns = 0.0;                // estimated duration of one run
 };
 
@@ -514,8 +516,9 @@ struct TaskBuilder
 
     TaskBuilder(uint32_t w, double s) : waves(w), simds(s), wrecs(w), wdesc(w), pending(w, 0), load(w) {}
 
-    // One level; bucket[type]: its records (each bend once).
-    void Level(const std::vector<uint4> (&bucket)[4])
+    // One level; bucket[type]: its records (each bend once).  all_quads: volumes, bends and edges
+    // on four lanes whatever the width.
+    void Level(const std::vector<uint4> (&bucket)[4], bool all_quads = false)
     {
         constexpr double kAlone = 1.15;
         uint32_t best = 0;
@@ -538,7 +541,7 @@ struct TaskBuilder
                 total += c * (double)tasks;
             }
             const double cost = std::max(kAlone * longest, total / simds);
-            if (!redundant && cost < best_cost)
+            if (all_quads ? m == 7 : !redundant && cost < best_cost)
             {
                 best_cost = cost;
                 best = m;
@@ -590,16 +593,18 @@ struct TaskBuilder
         ns += 170.0 + 2.25 * (tasks ? best_cost : 0.0);
     }
 
-    // Appends the program to `out`: its records, descriptors and `waves` heads.
+    // Appends the program to `out`: its records, descriptors and `waves` + 1 heads.
     void Finish(TaskProgram &out)
     {
         for (uint32_t w = 0; w < waves; ++w)
         {
+            out.desc.insert(out.desc.end(), kDescPad, 0u);
             out.heads.push_back(make_uint4((uint32_t)out.desc.size(), (uint32_t)wdesc[w].size(), (uint32_t)out.recs.size(), pending[w]));
             out.recs.insert(out.recs.end(), wrecs[w].begin(), wrecs[w].end());
             out.desc.insert(out.desc.end(), wdesc[w].begin(), wdesc[w].end());
             out.desc.insert(out.desc.end(), kDescPad, 0u);
         }
+        out.heads.push_back(make_uint4(0u, 0u, (uint32_t)out.recs.size(), 0u));
         out.recs.push_back(make_uint4(0u, 0u, 0u, 0u));     // read, not used, behind a task's records
         out.ns += ns;
     }
@@ -3198,11 +3203,14 @@ struct xpbd_rollout
     DevBuf<uint32_t> lvl;
     DevBuf<float4> x0;
     DevBuf<RolloutBodyDev> bodies;
-    DevBuf<float4> ckpt_x, ckpt_v, seg_x, seg_v, vel, prev, rec_tape, adj_x, adj_v;
+    DevBuf<uint4> task_recs, task_heads;
+    DevBuf<uint32_t> task_desc;
+    DevBuf<float4> ckpt_x, ckpt_v, seg_x, seg_v, vel, prev, tape, adj_x, adj_v;
     DevBuf<double> vel64, prev64;
     RolloutDev dev{};
     uint32_t total_nv = 0, total_ne = 0;
     uint32_t lds_f32 = 0, lds_f64 = 0, lds_bwd = 0;
+    bool bends = false;         // some body has dihedral bends
     bool has_forward = false;
 
     ~xpbd_rollout()
@@ -3213,6 +3221,9 @@ struct xpbd_rollout
 };
 
 namespace {
+// Largest segment tape of a rollout (the GPU has 288 GB)
+constexpr size_t kTapeBytes = (size_t)8 << 30;
+
 // The caller's stream as given: NULL is the default (null) stream, as in torch.
 hipStream_t StreamOf(xpbd_rollout *, void *stream) { return (hipStream_t)stream; }
 }
@@ -3231,6 +3242,14 @@ int xpbd_rollout_create(xpbd_context *ctx, const xpbd_rollout_desc *d, xpbd_roll
     std::vector<uint32_t> lvl;
     std::vector<float4> x0;
     std::vector<RolloutBodyDev> bodies(d->num_bodies);
+    TaskProgram tp;
+    struct TaskFirst { size_t recs, desc, heads; };
+    std::vector<TaskFirst> first(d->num_bodies);
+    size_t tape = 0;            // float4 of one sub-step's tape
+    for (uint32_t b = 0; b < d->num_bodies; ++b)
+        if (d->settings[b])
+            r->bends |= d->settings[b]->num_bends > 0;
+    const uint32_t waves = rollout_waves(r->bends);
     for (uint32_t b = 0; b < d->num_bodies; ++b)
     {
         xpbd_settings *s = d->settings[b];
@@ -3249,7 +3268,7 @@ int xpbd_rollout_create(xpbd_context *ctx, const xpbd_rollout_desc *d, xpbd_roll
         B.num_edges = ne;
         B.voff = r->total_nv;
         B.eoff = r->total_ne;
-        B.rbase = (uint32_t)recs.size();
+        const size_t rbase = recs.size();
         B.nlev = (uint32_t)s->host_level_begin.size() - 1;
         B.num_records = (uint32_t)s->host_recs.size();
         B.lvl = reinterpret_cast<const uint32_t *>((uintptr_t)lvl.size());     // index until uploaded
@@ -3260,12 +3279,10 @@ int xpbd_rollout_create(xpbd_context *ctx, const xpbd_rollout_desc *d, xpbd_roll
         B.vf_list = s->vf_list.p;
         for (uint32_t L : s->host_level_begin)
             lvl.push_back(L);                       // relative to the body's first record
-        B.edges_only = 1u;
+        B.edges_only = s->num_volumes + s->num_bends + s->num_lras == 0 ? 1u : 0u;
         for (size_t k = 0; k < s->host_recs.size(); ++k)
         {
             uint4 q = s->host_recs[k];
-            if (q.x != kNopRecordHost && ((q.x >> 14) & 3u) != kTypeEdge)
-                B.edges_only = 0u;
             if (q.x != kNopRecordHost && ((q.x >> 14) & 3u) != kTypeVolume && ((q.x >> 14) & 3u) != kTypeBend)
             {
                 // edges: their index in the body (for the compliance parameters) and a compliance
@@ -3275,6 +3292,42 @@ int xpbd_rollout_create(xpbd_context *ctx, const xpbd_rollout_desc *d, xpbd_roll
                 q.w = 0u;
             }
             recs.push_back(q);
+        }
+        B.recs = reinterpret_cast<const uint4 *>((uintptr_t)rbase);
+        // task program of the float passes; bodies of the same settings share it but for the
+        // records, which hold each body's compliances
+        {
+            TaskProgram own;
+            const uint32_t same = b > 0 && d->settings[b - 1] == s ? b - 1 : b;
+            if (same == b)
+            {
+                TaskBuilder builder(waves, 4.0);
+                std::vector<uint4> bucket[4];
+                const std::vector<uint4> body_recs(recs.begin() + rbase, recs.end());
+                for (size_t L = 0; L + 1 < s->host_level_begin.size(); ++L)
+                {
+                    LevelBuckets(body_recs, s->host_level_begin[L], s->host_level_begin[L + 1], bucket);
+                    builder.Level(bucket, true);
+                }
+                builder.Finish(own);
+                first[b] = { tp.recs.size(), tp.desc.size(), tp.heads.size() };
+                B.num_task_records = (uint32_t)own.recs.size() - 1u;
+                tp.recs.insert(tp.recs.end(), own.recs.begin(), own.recs.end());
+                tp.desc.insert(tp.desc.end(), own.desc.begin(), own.desc.end());
+                tp.heads.insert(tp.heads.end(), own.heads.begin(), own.heads.end());
+            }
+            else
+            {
+                first[b] = { tp.recs.size(), first[same].desc, first[same].heads };
+                B.num_task_records = bodies[same].num_task_records;
+                const size_t n = B.num_task_records + 1u;
+                tp.recs.resize(first[b].recs + n);
+                std::copy_n(tp.recs.begin() + first[same].recs, n, tp.recs.begin() + first[b].recs);
+            }
+            // edges and LRAs keep one float4 per record and sub-step, volumes and bends three
+            B.tape_stride = s->num_volumes + s->num_bends > 0 ? 3u : 1u;
+            B.tape_offset = tape;
+            tape += (size_t)B.tape_stride * (B.num_task_records + 1u);
         }
         for (const VertexRec &v : s->vertices)
             x0.push_back(make_float4(v.pos[0], v.pos[1], v.pos[2], v.inv_mass));
@@ -3287,9 +3340,16 @@ int xpbd_rollout_create(xpbd_context *ctx, const xpbd_rollout_desc *d, xpbd_roll
     HIP_TRY(r->recs.upload(recs));
     HIP_TRY(r->lvl.upload(lvl));
     HIP_TRY(r->x0.upload(x0));
-    for (RolloutBodyDev &B : bodies)
+    HIP_TRY(r->task_recs.upload(tp.recs));
+    HIP_TRY(r->task_desc.upload(tp.desc));
+    HIP_TRY(r->task_heads.upload(tp.heads));
+    for (uint32_t b = 0; b < d->num_bodies; ++b)
     {
-        B.recs = r->recs.p + B.rbase;
+        RolloutBodyDev &B = bodies[b];
+        B.task_recs = r->task_recs.p + first[b].recs;
+        B.task_desc = r->task_desc.p + first[b].desc;
+        B.task_heads = r->task_heads.p + first[b].heads;
+        B.recs = r->recs.p + (uintptr_t)B.recs;
         B.lvl = r->lvl.p + (uintptr_t)B.lvl;
         B.x0 = r->x0.p + B.voff;
     }
@@ -3298,10 +3358,14 @@ int xpbd_rollout_create(xpbd_context *ctx, const xpbd_rollout_desc *d, xpbd_roll
     const size_t nv = r->total_nv;
     const size_t seg_sub = (size_t)d->checkpoint_interval * d->num_iterations;
     HIP_TRY(r->ckpt_x.alloc(num_ckpt * nv)); HIP_TRY(r->ckpt_v.alloc(num_ckpt * nv));
-    HIP_TRY(r->seg_x.alloc(seg_sub * nv)); HIP_TRY(r->seg_v.alloc(seg_sub * nv));
+    HIP_TRY(r->seg_x.alloc((seg_sub + 1) * nv)); HIP_TRY(r->seg_v.alloc(seg_sub * nv));
     HIP_TRY(r->vel.alloc(nv)); HIP_TRY(r->prev.alloc(nv));
     HIP_TRY(r->vel64.alloc(4 * nv)); HIP_TRY(r->prev64.alloc(4 * nv));
-    HIP_TRY(r->rec_tape.alloc(4 * std::max<size_t>(recs.size(), 1)));
+    // The tape of a whole segment when it fits the budget (the adjoint then needs no second
+    // forward sweep of every sub-step), else of one sub-step.
+    const uint32_t tape_subs = std::min<size_t>(seg_sub, (size_t)d->frames * d->num_iterations) * tape * sizeof(float4) <= kTapeBytes
+                                   ? (uint32_t)std::min<size_t>(seg_sub, (size_t)d->frames * d->num_iterations) : 1u;
+    HIP_TRY(r->tape.alloc(tape * tape_subs));
     HIP_TRY(r->adj_x.alloc(nv)); HIP_TRY(r->adj_v.alloc(nv));
     RolloutDev &R = r->dev;
     R.bodies = r->bodies.p;
@@ -3317,7 +3381,7 @@ int xpbd_rollout_create(xpbd_context *ctx, const xpbd_rollout_desc *d, xpbd_roll
     R.gravity_factor = d->gravity_factor;
     R.ckpt_x = r->ckpt_x.p; R.ckpt_v = r->ckpt_v.p; R.seg_x = r->seg_x.p; R.seg_v = r->seg_v.p;
     R.vel = r->vel.p; R.prev = r->prev.p; R.vel64 = r->vel64.p; R.prev64 = r->prev64.p;
-    R.rec_tape = r->rec_tape.p; R.adj_x = r->adj_x.p; R.adj_v = r->adj_v.p;
+    R.tape = r->tape.p; R.tape_size = tape; R.tape_subs = tape_subs; R.adj_x = r->adj_x.p; R.adj_v = r->adj_v.p;
     *out = r.release();
     return XPBD_OK;
 }
@@ -3346,7 +3410,7 @@ int xpbd_rollout_forward(xpbd_rollout *r, const float *compliance, const float *
     if (!r || !compliance || !velocity || !positions)
         return Fail(XPBD_E_INVALID, "null argument");
     HIP_TRY(hipSetDevice(r->ctx->device));
-    HIP_TRY(launch_rollout_forward_f32(r->dev, compliance, velocity, positions, r->lds_f32, StreamOf(r, stream)));
+    HIP_TRY(launch_rollout_forward_f32(r->dev, r->bends, compliance, velocity, positions, r->lds_f32, StreamOf(r, stream)));
     r->has_forward = true;
     return XPBD_OK;
 }
@@ -3359,7 +3423,7 @@ int xpbd_rollout_forward_noalloc(xpbd_rollout *r, const float *compliance, const
         return Fail(XPBD_E_CAPACITY, "rollout has " + std::to_string(r->total_nv) + " vertices; the allocation-free forward pass holds at most "
                                          + std::to_string(rollout_noalloc_max_vertices()));
     HIP_TRY(hipSetDevice(r->ctx->device));
-    HIP_TRY(launch_rollout_forward_f32_noalloc(r->ctx->device, r->dev, compliance, velocity, positions, r->lds_f32, StreamOf(r, stream)));
+    HIP_TRY(launch_rollout_forward_f32_noalloc(r->ctx->device, r->dev, r->bends, compliance, velocity, positions, r->lds_f32, StreamOf(r, stream)));
     r->has_forward = true;
     return XPBD_OK;
 }
@@ -3382,7 +3446,7 @@ int xpbd_rollout_backward(xpbd_rollout *r, const float *grad_positions, float *g
     if (!r->has_forward)
         return Fail(XPBD_E_INVALID, "backward needs a float forward pass first");
     HIP_TRY(hipSetDevice(r->ctx->device));
-    HIP_TRY(launch_rollout_backward(r->dev, grad_positions, grad_compliance, grad_velocity, r->lds_bwd, StreamOf(r, stream)));
+    HIP_TRY(launch_rollout_backward(r->dev, r->bends, grad_positions, grad_compliance, grad_velocity, r->lds_bwd, StreamOf(r, stream)));
     return XPBD_OK;
 }
 

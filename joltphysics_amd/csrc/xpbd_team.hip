@@ -270,12 +270,12 @@ __global__ __launch_bounds__(kTeamBlock) void team_kernel(
                 const RecordCtx rc{ B.skin, B.skin_base, (float)(it + 1) / (float)iterations, nullptr, nullptr, nullptr };
                 auto run_window = [&](uint32_t w) {
                     const WindowDev W = S.windows[w];
-                    TaskStream tasks;
-                    tasks.begin(S.task_recs, S.task_desc, S.task_heads + (size_t)w * kStreamedWaves + wave, (uint32_t)lane);
+                    TaskStream<> tasks;
+                    tasks.begin(S.task_recs, S.task_desc, S.task_heads + (size_t)w * (kStreamedWaves + 1u) + wave, (uint32_t)lane);
                     for (uint32_t j = tid; j < W.vcount; j += kTeamBlock)
                         X[j] = P[S.vlist[W.vbegin + j]];
                     __syncthreads();
-                    tasks.run(X, inv_dt_sq, (uint32_t)lane, NoSkip(), rc);
+                    run_tasks(tasks, X, inv_dt_sq, (uint32_t)lane, NoSkip(), rc);
                     for (uint32_t j = tid; j < W.vcount; j += kTeamBlock)
                         P[S.vlist[W.vbegin + j]] = X[j];
                     __syncthreads();

@@ -41,7 +41,7 @@ struct SettingsDev
     const uint32_t *lvl;        // absolute record offset of each level start, nlev+1 per window
     const WindowDev *windows;   // parallel-group windows, then tail windows
     // gathered windows without rods run as task programs of kStreamedWaves wavefronts: records,
-    // descriptors, and kStreamedWaves heads per window
+    // descriptors, and kStreamedWaves + 1 heads per window
     const uint4 *task_recs;
     const uint32_t *task_desc;
     const uint4 *task_heads;
@@ -242,7 +242,7 @@ struct BundleDev
 {
     const uint4 *recs;          // task program of the merged levels (vertex numbers are bundle-local)
     const uint32_t *desc;
-    const uint4 *heads;         // one per wavefront
+    const uint4 *heads;         // one per wavefront, and one behind them
     const BundleBodyDev *bodies;
     uint32_t num_bodies;
     uint32_t nv;                // vertices of all bodies of the bundle
@@ -274,13 +274,20 @@ struct RolloutBodyDev
     uint32_t nlev, num_records;
     uint32_t nv, num_edges;
     uint32_t voff, eoff;        // first vertex / edge in the concatenated arrays
-    uint32_t rbase;             // first record slot in the record tape
     const float4 *x0;           // initial positions + inverse mass
     // pressure (num_faces 0: none): faces (3 vertices each) and vertex -> face lists in face order
     const uint32_t *faces, *vf_begin, *vf_list;
     uint32_t num_faces;
     float pressure;
     uint32_t edges_only;        // 1: every record is an edge (the level passes skip the type dispatch)
+    // task program of the float passes (volumes, bends and edges on four lanes, an edge's y its
+    // index in the body, its w its compliance) and its tape
+    uint4 *task_recs;
+    const uint32_t *task_desc;
+    const uint4 *task_heads;
+    uint32_t num_task_records;
+    uint32_t tape_stride;       // float4 per record and sub-step
+    size_t tape_offset;         // first float4 of the body in a sub-step's tape
 };
 
 struct RolloutDev
@@ -291,10 +298,14 @@ struct RolloutDev
     float gravity[3];           // world gravity (bodies have identity rotation, so also body-local)
     float gravity_factor;
     float4 *ckpt_x, *ckpt_v;    // (x + inverse mass, v) at frames 0, interval, 2 interval, ...
-    float4 *seg_x, *seg_v;      // state at every sub-step start of the segment being reversed
+    float4 *seg_x, *seg_v;      // state at every sub-step start of the segment being reversed (seg_x: and its end)
     float4 *vel, *prev;         // float forward state
     double *vel64, *prev64;     // double forward state (4 per vertex)
-    float4 *rec_tape;           // 4 per record: pre-projection positions (+ inverse mass) of its vertices
+    // what each record's adjoint needs of its projection, per sub-step: an edge {delta, length}, an
+    // LRA {delta, squared length}, a volume or bend {x0, x1, x2, x3} per component
+    float4 *tape;
+    size_t tape_size;           // float4 per sub-step
+    uint32_t tape_subs;         // sub-steps held: a whole segment, or 1
     float4 *adj_x, *adj_v;      // adjoint state
 };
 
