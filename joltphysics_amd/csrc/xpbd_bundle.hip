@@ -32,7 +32,8 @@ struct BodyLocal
     float dgx, dgy, dgz;        // displacement due to gravity
     float restitution_threshold, max_lin_sq;
     float delta[3];             // recentring of this step
-    float six_volume;           // pressure
+    float coefficient;          // pressure: p h / six-volume
+    uint32_t inflated;          // the six-volume is positive: pressure acts
     uint32_t num_leaves;
     uint32_t num_dyn_leaves;    // leaves of dynamic colliders this step
     uint32_t num_dynamic;       // dynamic colliders of the context
@@ -43,10 +44,7 @@ struct BodyLocal
     uint32_t ran;               // the body was active at the start of this step
     DynStateDev *dyn;           // the body's row of dynamic-collider states
     const float4 *pair;         // the body's per-collider contact settings, or null
-    uint32_t nf;
-    const uint32_t *faces;
-    const uint32_t *vf_begin;
-    const uint32_t *vf_list;
+    uint32_t nf;                // faces under pressure
 };
 
 struct BundleLds
@@ -126,7 +124,6 @@ __device__ __forceinline__ void bundle_update(
         L.gravity_factor = B.gravity_factor; L.vertex_radius = B.vertex_radius;
         L.update_position = B.update_position; L.allow_sleeping = B.allow_sleeping;
         L.nf = B.pressure > 0.0f ? B.s.num_faces : 0u;
-        L.faces = B.s.faces; L.vf_begin = B.s.vf_begin; L.vf_list = B.s.vf_list;
         L.dyn = B.dyn;
         L.pair = B.pair;
         L.report_cleared = 0;
@@ -289,70 +286,6 @@ __device__ __forceinline__ void bundle_update(
                 }
             }
 
-            // ---- ApplyPressure (SoftBodyMotionProperties.cpp:291-323)
-            auto apply_pressure = [&]() {
-                // GetVolumeTimesSix: a sequential sum in face order, one wavefront per
-                // body.  The lanes compute the terms of 64 faces at a time and the sum
-                // takes them in lane order, so the additions happen in face order.
-                for (uint32_t b = wave; b < nb; b += (BLOCK / kWave))
-                {
-                    const BodyLocal &L = loc[b];
-                    if (L.nf == 0 || !st[b].active)
-                        continue;
-                    const uint32_t voff = G.bodies[b].voff;
-                    float six = 0.0f;
-                    for (uint32_t f0 = 0; f0 < L.nf; f0 += kWave)
-                    {
-                        const uint32_t f = f0 + (uint32_t)lane;
-                        float term = 0.0f;
-                        if (f < L.nf)
-                        {
-                            V3 x1 = xyz(pget(X, voff + L.faces[3 * f])), x2 = xyz(pget(X, voff + L.faces[3 * f + 1])), x3 = xyz(pget(X, voff + L.faces[3 * f + 2]));
-                            term = dot(cross(x1, x2), x3);
-                        }
-                        const uint32_t count = L.nf - f0 < (uint32_t)kWave ? L.nf - f0 : (uint32_t)kWave;
-                        for (uint32_t k = 0; k < count; ++k)
-                            six += __int_as_float(__builtin_amdgcn_readlane(__float_as_int(term), k));
-                    }
-                    if (lane == 0)
-                        loc[b].six_volume = six;
-                }
-                __syncthreads();
-                for (uint32_t b = 0; b < nb; ++b)
-                {
-                    const BodyLocal &L = loc[b];
-                    if (L.nf == 0 || !st[b].active || !(L.six_volume > 0.0f))
-                        continue;
-                    const BundleBodyDev bb = G.bodies[b];
-                    const float coefficient = L.pressure * L.dt_sub / L.six_volume;
-                    for (uint32_t f = tid; f < L.nf; f += BLOCK)
-                    {
-                        V3 x1 = xyz(pget(X, bb.voff + L.faces[3 * f])), x2 = xyz(pget(X, bb.voff + L.faces[3 * f + 1])), x3 = xyz(pget(X, bb.voff + L.faces[3 * f + 2]));
-                        V3 impulse = coefficient * cross(x2 - x1, x3 - x1);
-                        G.face_scratch[bb.face_off + f] = make_float4(impulse.x, impulse.y, impulse.z, 0.0f);
-                    }
-                }
-                sync_global();
-                for (uint32_t i = tid; i < nv; i += BLOCK)
-                {
-                    const uint32_t b = body_of(i);
-                    const BodyLocal &L = loc[b];
-                    if (L.nf == 0 || !st[b].active || !(L.six_volume > 0.0f))
-                        continue;
-                    const BundleBodyDev bb = G.bodies[b];
-                    const uint32_t li = i - bb.voff;
-                    uint32_t fb = L.vf_begin[li], fe = L.vf_begin[li + 1];
-                    if (fb == fe)
-                        continue;
-                    float w = pget(X, i).w;
-                    V3 v = xyz(G.v[i]);
-                    for (uint32_t k = fb; k < fe; ++k)
-                        v = v + w * xyz(G.face_scratch[bb.face_off + L.vf_list[k]]);
-                    G.v[i] = f4(v, 0.0f);
-                }
-                __syncthreads();
-            };
-
             // ---- IntegratePositions (SoftBodyMotionProperties.cpp:325-350)
             auto integrate_vertex = [&](uint32_t i, const BodyLocal &L, float4 p, V3 v) {
                 if (p.w > 0.0f)
@@ -367,15 +300,65 @@ __device__ __forceinline__ void bundle_update(
                 G.v[i] = f4(v, 0.0f);
             };
 
+            // ---- ApplyPressure (SoftBodyMotionProperties.cpp:291-323), then IntegratePositions, of
+            // every body, or only of those under pressure (the others have integrated already).
+            // The whole workgroup forms every face's term and normal, one wavefront per body sums
+            // the terms in face order, then each vertex adds its faces' impulses in face order
+            // and integrates.  A 2,562-vertex sphere alone in its workgroup takes 40 us a
+            // sub-step, 330 when the wavefront that sums also formed the terms.
+            auto apply_pressure_and_integrate = [&](bool all) {
+                for (uint32_t f = tid; f < G.num_faces; f += BLOCK)
+                {
+                    const uint2 q = G.faces[f];
+                    const V3 x1 = xyz(pget(X, q.x & 0x3fffu)), x2 = xyz(pget(X, (q.x >> 14) & 0x3fffu)), x3 = xyz(pget(X, q.y & 0x3fffu));
+                    G.face_terms[f] = dot(cross(x1, x2), x3);
+                    G.face_normals[f] = f4(cross(x2 - x1, x3 - x1), 0.0f);
+                }
+                sync_global();
+                for (uint32_t b = wave; b < nb; b += (BLOCK / kWave))
+                {
+                    const BodyLocal &L = loc[b];
+                    if (L.nf == 0 || !st[b].active)
+                        continue;
+                    const float six_volume = ordered_sum(G.face_terms + G.bodies[b].face_off, L.nf, lane);     // GetVolumeTimesSix
+                    if (lane == 0)
+                        loc[b].coefficient = six_volume > 0.0f ? L.pressure * L.dt_sub / six_volume : 0.0f;
+                    if (lane == 0)
+                        loc[b].inflated = six_volume > 0.0f ? 1u : 0u;
+                }
+                __syncthreads();
+                for (uint32_t i = tid; i < nv; i += BLOCK)
+                {
+                    const uint32_t b = body_of(i);
+                    const BodyLocal &L = loc[b];
+                    if (!st[b].active || !(all || L.nf > 0))
+                        continue;
+                    const float4 p = pget(X, i);
+                    V3 v = xyz(G.v[i]);
+                    if (L.nf > 0 && L.inflated)
+                    {
+                        const uint32_t fe = G.vf_begin[i + 1];
+                        for (uint32_t k = G.vf_begin[i]; k < fe; ++k)
+                            v = v + p.w * (L.coefficient * xyz(G.face_normals[G.vf_list[k]]));
+                    }
+                    integrate_vertex(i, L, p, v);
+                }
+                // the next terms overwrite what the vertices of other wavefronts read
+                __syncthreads();
+            };
+
             if (G.has_pressure)
-                apply_pressure();
-            for (uint32_t i = tid; i < nv; i += BLOCK)
+                apply_pressure_and_integrate(true);
+            else
             {
-                const uint32_t b = body_of(i);
-                if (st[b].active)
-                    integrate_vertex(i, loc[b], pget(X, i), xyz(G.v[i]));
+                for (uint32_t i = tid; i < nv; i += BLOCK)
+                {
+                    const uint32_t b = body_of(i);
+                    if (st[b].active)
+                        integrate_vertex(i, loc[b], pget(X, i), xyz(G.v[i]));
+                }
+                __syncthreads();
             }
-            __syncthreads();
 
             for (uint32_t it = 0; it < iterations; ++it)
             {
@@ -499,17 +482,7 @@ __device__ __forceinline__ void bundle_update(
                 }
                 __syncthreads();
                 if (!last && G.has_pressure)
-                {
-                    apply_pressure();
-                    for (uint32_t i = tid; i < nv; i += BLOCK)
-                    {
-                        const uint32_t b = body_of(i);
-                        const BodyLocal &L = loc[b];
-                        if (st[b].active && L.nf > 0)
-                            integrate_vertex(i, L, pget(X, i), xyz(G.v[i]));
-                    }
-                    __syncthreads();
-                }
+                    apply_pressure_and_integrate(false);
             }
 
             // the reductions read velocities other wavefronts stored

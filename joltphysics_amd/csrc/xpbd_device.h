@@ -2018,6 +2018,38 @@ __device__ __forceinline__ float wave_max(float v)
     for (int o = 32; o > 0; o >>= 1) { float u = __shfl_xor(v, o, kWave); v = u > v ? u : v; }
     return v;
 }
+// ((t[0] + t[1]) + t[2]) + ... of n terms in order, by one wavefront, the result in every lane.
+// A chain of n dependent additions, so what counts is the instructions per term: each lane of a
+// 16-lane row holds one of 16 terms and one addition takes it as a DPP row broadcast, 5 cycles a
+// term (a readlane loop takes about 30); the next 64 terms load meanwhile.
+template <int K>
+__device__ __forceinline__ float add_row(float acc, float t)
+{
+    if constexpr (K < 16)
+        return add_row<K + 1>(__int_as_float(__builtin_amdgcn_mov_dpp(__float_as_int(t), 0x150 + K, 0xf, 0xf, true)) + acc, t);  // row_newbcast:K
+    else
+        return acc;
+}
+__device__ __forceinline__ float ordered_sum(const float *terms, uint32_t n, uint32_t lane)
+{
+    float acc = 0.0f;
+    const uint32_t k = lane & 15u;
+    auto term = [&](uint32_t f) { return f < n ? terms[f] : 0.0f; };    // adding +0 changes no partial sum
+    float t0 = term(k), t1 = term(k + 16u), t2 = term(k + 32u), t3 = term(k + 48u);
+    for (uint32_t f = 0; f < n; f += 64u)
+    {
+        const float u0 = t0, u1 = t1, u2 = t2, u3 = t3;
+        t0 = term(f + 64u + k);
+        t1 = term(f + 80u + k);
+        t2 = term(f + 96u + k);
+        t3 = term(f + 112u + k);
+        acc = add_row<0>(acc, u0);
+        acc = add_row<0>(acc, u1);
+        acc = add_row<0>(acc, u2);
+        acc = add_row<0>(acc, u3);
+    }
+    return acc;
+}
 __device__ __forceinline__ float wave_sum(float v)
 {
     for (int o = 32; o > 0; o >>= 1) v += __shfl_xor(v, o, kWave);

@@ -401,7 +401,7 @@ template <> __device__ __forceinline__ R4<double> *state_prev<double>(const Roll
 
 // ApplyPressure (SoftBodyMotionProperties.cpp:291-323) on the sub-step start positions X (LDS)
 // and the velocities V, with the operation order of the update kernel: GetVolumeTimesSix
-// (:107-118) summed in face order by one lane from per-face terms (terms: num_faces + 2 slots),
+// (:107-118) summed in face order (by one wavefront in float) from per-face terms (terms: num_faces + 2 slots),
 // then each vertex adds its faces' impulses w * c * (x2 - x1) x (x3 - x1) in face order.
 template <int BLOCK, class T>
 __device__ __forceinline__ void pressure_apply(const RolloutBodyDev &B, const StepConstants<T> &K, const R4<T> *X, R4<T> *V,
@@ -414,7 +414,16 @@ __device__ __forceinline__ void pressure_apply(const RolloutBodyDev &B, const St
         terms[f] = rdot(rcross(xyz3(X[t[0]]), xyz3(X[t[1]])), xyz3(X[t[2]]));
     }
     __syncthreads();
-    if (tid == 0)
+    if constexpr (sizeof(T) == 4)
+    {
+        if (tid < (uint32_t)kWave)
+        {
+            const float six_volume = ordered_sum(terms, nf, tid);
+            if (tid == 0)
+                terms[nf] = six_volume;
+        }
+    }
+    else if (tid == 0)
     {
         T six_volume = (T)0;
         for (uint32_t f = 0; f < nf; ++f)
@@ -473,12 +482,11 @@ __device__ __forceinline__ void pressure_adjoint(const RolloutBodyDev &B, float 
     if (tid == 0)
         terms[nf + 1] = 0.0f;
     __syncthreads();
-    if (tid == 0)
+    if (tid < (uint32_t)kWave)
     {
-        float six_volume = 0.0f;
-        for (uint32_t f = 0; f < nf; ++f)
-            six_volume += terms[f];
-        terms[nf] = six_volume;
+        const float six_volume = ordered_sum(terms, nf, tid);
+        if (tid == 0)
+            terms[nf] = six_volume;
     }
     __syncthreads();
     const float S = terms[nf];

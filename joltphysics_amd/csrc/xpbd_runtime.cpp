@@ -125,6 +125,7 @@ struct xpbd_settings
     xpbd_context *ctx = nullptr;
     int refcount = 1;
     uint32_t num_vertices = 0, num_faces = 0;
+    std::vector<uint32_t> host_faces, host_vf_begin, host_vf_list;     // host copies of faces, vf_begin, vf_list
     std::vector<VertexRec> vertices;        // host copy for body creation
     DevBuf<uint4> recs;
     DevBuf<uint32_t> lvl;
@@ -201,7 +202,10 @@ struct BundleHost
     DevBuf<uint4> recs, heads;
     DevBuf<uint32_t> desc;
     DevBuf<BundleBodyDev> table;
-    DevBuf<float4> x, v, prev, plane, report, face_scratch;
+    DevBuf<float4> x, v, prev, plane, report, face_normals;
+    DevBuf<uint2> faces;
+    DevBuf<uint32_t> vf_begin, vf_list;
+    DevBuf<float> face_terms;
     DevBuf<int32_t> idx, contact;
     DevBuf<unsigned char> leaves_full, leaves;
     BundleDev dev{};
@@ -1176,6 +1180,9 @@ int BuildSchedule(const xpbd_settings_desc &d, xpbd_settings &s, int32_t schedul
                 vf_list[fill[faces[f].v[j]]++] = f;
     }
 
+    s.host_faces = f3;
+    s.host_vf_begin = vf_begin;
+    s.host_vf_list = vf_list;
     hipError_t e;
     if (s.host_schedule)
     {
@@ -1660,13 +1667,42 @@ int BuildLayout(xpbd_context *ctx)
         }
         HIP_TRY(bh.leaves_full.alloc((size_t)std::max(1u, nb * nc) * bundle_leaf_bytes()));
         HIP_TRY(bh.leaves.alloc((size_t)std::max(1u, nb * nc) * bundle_leaf_bytes()));
-        HIP_TRY(bh.face_scratch.alloc(std::max(1u, P.foff)));
+        if (P.has_pressure)
+        {
+            std::vector<uint2> faces;
+            std::vector<uint32_t> vf_begin(1, 0u), vf_list;
+            faces.reserve(P.foff);
+            for (uint32_t j = 0; j < nb; ++j)
+            {
+                const Body &b = *ctx->bodies[bh.bodies[j]];
+                const xpbd_settings &st = *b.settings;
+                const bool pressed = b.dev.pressure > 0.0f && st.num_faces > 0;
+                const uint32_t first = (uint32_t)faces.size(), o = P.voffs[j];
+                if (pressed)
+                    for (uint32_t f = 0; f < st.num_faces; ++f)
+                        faces.push_back(make_uint2((st.host_faces[3 * f] + o) | (st.host_faces[3 * f + 1] + o) << 14,
+                                                   (st.host_faces[3 * f + 2] + o) | j << 16));
+                for (uint32_t i = 0; i < b.nv; ++i)
+                {
+                    if (pressed)
+                        for (uint32_t q = st.host_vf_begin[i]; q < st.host_vf_begin[i + 1]; ++q)
+                            vf_list.push_back(first + st.host_vf_list[q]);
+                    vf_begin.push_back((uint32_t)vf_list.size());
+                }
+            }
+            HIP_TRY(bh.faces.upload(faces));
+            HIP_TRY(bh.vf_begin.upload(vf_begin));
+            HIP_TRY(bh.vf_list.upload(vf_list));
+            HIP_TRY(bh.face_normals.alloc(faces.size()));
+            HIP_TRY(bh.face_terms.alloc(faces.size()));
+        }
         BundleDev &d = bh.dev;
         d.recs = bh.recs.p; d.desc = bh.desc.p; d.heads = bh.heads.p;
         d.bodies = bh.table.p; d.num_bodies = nb; d.nv = voff;
         d.x = bh.x.p; d.v = bh.v.p; d.prev = bh.prev.p; d.plane = bh.plane.p; d.idx = bh.idx.p; d.contact = bh.contact.p;
         d.report = bh.report.p;
-        d.leaves_full = bh.leaves_full.p; d.leaves = bh.leaves.p; d.face_scratch = bh.face_scratch.p;
+        d.leaves_full = bh.leaves_full.p; d.leaves = bh.leaves.p; d.faces = bh.faces.p; d.num_faces = P.has_pressure ? P.foff : 0u; d.vf_begin = bh.vf_begin.p; d.vf_list = bh.vf_list.p;
+        d.face_normals = bh.face_normals.p; d.face_terms = bh.face_terms.p;
         d.has_pressure = P.has_pressure ? 1u : 0u;
         d.has_sleepers = P.has_sleepers ? 1u : 0u;
         d.iterations = P.iterations;

@@ -250,7 +250,14 @@ struct BundleDev
     int32_t *idx, *contact;
     void *leaves_full;          // num_bodies x num_colliders Leaf: per-step candidate leaves
     void *leaves;               // num_bodies x num_colliders Leaf: compacted colliding list
-    float4 *face_scratch;       // pressure scratch, one slot per face of the bundle's pressure bodies
+    // pressure: the faces of the bundle's pressure bodies, body by body: {vertex 0 | vertex 1 << 14,
+    // vertex 2 | body << 16} (bundle-local); per bundle vertex its faces in face order (CSR); per face
+    // its normal (x2 - x1) x (x3 - x1) and its term of the six-volume
+    const uint2 *faces;
+    uint32_t num_faces;
+    const uint32_t *vf_begin, *vf_list;
+    float4 *face_normals;
+    float *face_terms;
     uint32_t has_pressure;
     uint32_t has_sleepers;
     uint32_t iterations;
