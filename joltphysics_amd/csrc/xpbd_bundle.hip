@@ -127,6 +127,7 @@ __device__ __forceinline__ void bundle_update(
         L.dyn = B.dyn;
         L.pair = B.pair;
         L.report_cleared = 0;
+        L.delta[0] = L.delta[1] = L.delta[2] = 0.0f;        // a body asleep from the start of the launch recentres by it
         L.skin_entries = B.skin ? B.skin + 4u * (size_t)B.skin_base : nullptr;
         L.sensor_hits = B.sensor_hits;
         L.num_sensors = B.sensor_hits ? B.num_sensors : 0u;
