@@ -34,6 +34,7 @@ hipError_t launch_team(bool ext, const BodyDev *bodies, BodyStateDev *states, co
                        uint32_t num_blocks, const ColliderDev *colliders, uint32_t num_colliders, uint32_t max_leaves,
                        uint32_t lds_bytes, float gx, float gy, float gz, float dt, int32_t steps, int32_t frames,
                        int32_t *error_flag, hipStream_t stream);
+hipError_t launch_readback(const ReadSources &s, uint32_t nv, ReadHeader *header, uint32_t *out, hipStream_t stream);
 hipError_t launch_skin(const float *joints, const SkinInvBindDev *inv_binds, uint32_t num_inv_binds, float *skin,
                        const SkinnedDev *recs, uint32_t num_recs, const uint32_t *normal_faces, const uint32_t *faces,
                        float4 *states, uint32_t nv, float4 *x, float4 *v, int32_t hard_skin_all, hipStream_t stream);
@@ -247,6 +248,9 @@ struct xpbd_context
     DevBuf<DynStateDev> d_dyn;      // bodies x num_dynamic
     uint32_t dyn_stride = 0;        // num_dynamic the rows of d_dyn are laid out for
     DevBuf<int32_t> d_error;
+    // pinned host memory a read-back packs a body into, at most twice what the largest read needed
+    unsigned char *h_read = nullptr;
+    size_t h_read_n = 0;
     float gravity[3] = { 0.0f, -9.81f, 0.0f };       // PhysicsSystem.h:392 default
     bool profiling = false;
     std::vector<std::pair<hipEvent_t, hipEvent_t>> events;
@@ -1860,6 +1864,8 @@ int xpbd_context_destroy(xpbd_context *ctx)
     (void)hipEventDestroy(ctx->elapsed_ready);
     if (ctx->h_elapsed)
         (void)hipHostFree(ctx->h_elapsed);
+    if (ctx->h_read)
+        (void)hipHostFree(ctx->h_read);
     for (int a = 0; a < ctx->num_aux; ++a)
     {
         (void)hipEventDestroy(ctx->join[a]);
@@ -2638,14 +2644,22 @@ int xpbd_update(xpbd_context *ctx, float dt, int32_t collision_steps, int32_t fr
     // are enough: the streamed bodies on the context stream, then the bundle
     // launches, largest LDS first.  With more groups than streams a group goes to
     // the stream with the least estimated work queued.
+    // An auxiliary stream joins in only when a group goes to it: an event record or wait costs the
+    // host and the queue several microseconds, and a single group needs none.
     const int num_aux = ctx->num_aux;
-    HIP_TRY(hipEventRecord(ctx->fork, ctx->stream));
-    for (int a = 0; a < num_aux; ++a)
-        HIP_TRY(hipStreamWaitEvent(ctx->aux[a], ctx->fork, 0));
+    if ((ctx->teams.empty() ? 0 : 1) + launches.size() + ctx->bundle_launches.size() > 1)
+        HIP_TRY(hipEventRecord(ctx->fork, ctx->stream));
+    bool forked[xpbd_context::kMaxAux + 1] = { true };      // the context stream itself
     const float gx = ctx->gravity[0], gy = ctx->gravity[1], gz = ctx->gravity[2];
     hipStream_t streams[xpbd_context::kMaxAux + 1] = { ctx->stream };
     for (int a = 0; a < num_aux; ++a) streams[a + 1] = ctx->aux[a];
     double queued[xpbd_context::kMaxAux + 1] = {};
+    auto fork_stream = [&](int q) -> hipError_t {
+        if (forked[q])
+            return hipSuccess;
+        forked[q] = true;
+        return hipStreamWaitEvent(streams[q], ctx->fork, 0);
+    };
     auto least_queued = [&]() {
         int best = 0;
         for (int q = 1; q <= num_aux; ++q)
@@ -2670,6 +2684,7 @@ int xpbd_update(xpbd_context *ctx, float dt, int32_t collision_steps, int32_t fr
     for (const Launch &l : launches)
     {
         const int q = ctx->teams.empty() ? 0 : least_queued();
+        HIP_TRY(fork_stream(q));
         HIP_TRY(launch_update(l.resident, l.staged, l.rods, ctx->ext_colliders, ctx->d_bodies.p, ctx->d_states.p, ctx->d_list.p + offset, (uint32_t)l.bodies.size(),
                               ctx->d_colliders.p, nc, l.max_leaves, l.lds, gx, gy, gz, dt, collision_steps, frames, ctx->d_error.p, streams[q]));
         offset += (uint32_t)l.bodies.size();
@@ -2683,11 +2698,14 @@ int xpbd_update(xpbd_context *ctx, float dt, int32_t collision_steps, int32_t fr
         const auto &L = *Lp;
         const int best = least_queued();
         queued[best] += std::max(L.cost, L.work / 256.0);
+        HIP_TRY(fork_stream(best));
         HIP_TRY(launch_bundles(L.block, L.uniform, ctx->ext_colliders, L.table.p, L.count, ctx->d_bodies.p, ctx->d_states.p, ctx->d_colliders.p, nc,
                                L.lds, gx, gy, gz, dt, collision_steps, frames, streams[best]));
     }
     for (int a = 0; a < num_aux; ++a)
     {
+        if (!forked[a + 1])
+            continue;
         HIP_TRY(hipEventRecord(ctx->join[a], ctx->aux[a]));
         HIP_TRY(hipStreamWaitEvent(ctx->stream, ctx->join[a], 0));
     }
@@ -2706,6 +2724,20 @@ int xpbd_update(xpbd_context *ctx, float dt, int32_t collision_steps, int32_t fr
     return XPBD_OK;
 }
 
+namespace {
+// The error of a finished update, from the device's flag (cleared where it was set)
+int CheckError(xpbd_context *ctx, int32_t err)
+{
+    if (!err)
+        return XPBD_OK;
+    HIP_TRY(hipMemset(ctx->d_error.p, 0, sizeof(int32_t)));
+    if (err & 4)
+        return Fail(XPBD_E_DEVICE, "a team of workgroups waited too long at a barrier (its members did not all run at once); "
+                                   "the update's results are invalid");
+    return Fail(XPBD_E_CAPACITY, "a body collided with more colliders than the leaf capacity");
+}
+} // namespace
+
 int xpbd_synchronize(xpbd_context *ctx)
 {
     if (!ctx)
@@ -2714,15 +2746,7 @@ int xpbd_synchronize(xpbd_context *ctx)
     HIP_TRY(hipStreamSynchronize(ctx->stream));
     int32_t err = 0;
     HIP_TRY(hipMemcpy(&err, ctx->d_error.p, sizeof(err), hipMemcpyDeviceToHost));
-    if (err)
-    {
-        HIP_TRY(hipMemset(ctx->d_error.p, 0, sizeof(int32_t)));
-        if (err & 4)
-            return Fail(XPBD_E_DEVICE, "a team of workgroups waited too long at a barrier (its members did not all run at once); "
-                                       "the update's results are invalid");
-        return Fail(XPBD_E_CAPACITY, "a body collided with more colliders than the leaf capacity");
-    }
-    return XPBD_OK;
+    return CheckError(ctx, err);
 }
 
 int xpbd_body_read(xpbd_context *ctx, int32_t body, float *pos, float *prev, float *vel, float *plane, int32_t *shape_idx,
@@ -2730,33 +2754,47 @@ int xpbd_body_read(xpbd_context *ctx, int32_t body, float *pos, float *prev, flo
 {
     if (!ctx || body < 0 || body >= (int32_t)ctx->bodies.size())
         return Fail(XPBD_E_INVALID, "invalid body");
-    int rc = xpbd_synchronize(ctx);
-    if (rc != XPBD_OK)
-        return rc;
-    rc = PullStates(ctx);
-    if (rc != XPBD_OK)
-        return rc;
+    HIP_TRY(hipSetDevice(ctx->device));
     Body &b = *ctx->bodies[body];
-    const uint32_t nv = b.nv;
-    std::vector<float4> tmp(nv);
-    auto get3 = [&](const float4 *src, float *dst, int comps) -> int {
-        if (!dst)
-            return XPBD_OK;
-        HIP_TRY(hipMemcpy(tmp.data(), src, sizeof(float4) * nv, hipMemcpyDeviceToHost));
-        for (uint32_t i = 0; i < nv; ++i)
-        {
-            dst[comps * i] = tmp[i].x; dst[comps * i + 1] = tmp[i].y; dst[comps * i + 2] = tmp[i].z;
-            if (comps == 4) dst[comps * i + 3] = tmp[i].w;
-        }
-        return XPBD_OK;
-    };
-    if ((rc = get3(b.dev.x, pos, 3)) != XPBD_OK || (rc = get3(b.dev.prev, prev, 3)) != XPBD_OK || (rc = get3(b.dev.v, vel, 3)) != XPBD_OK
-        || (rc = get3(b.dev.plane, plane, 4)) != XPBD_OK)
+    const size_t nv = b.nv;
+    const size_t words = nv * ((pos ? 3 : 0) + (prev ? 3 : 0) + (vel ? 3 : 0) + (plane ? 4 : 0) + (shape_idx ? 1 : 0) + (contact ? 1 : 0));
+    constexpr size_t kHeader = (sizeof(ReadHeader) + 255) / 256 * 256;
+    const size_t need = kHeader + 4 * words;
+    if (ctx->h_read_n < need)
+    {
+        const size_t size = std::max(need, 2 * ctx->h_read_n);
+        if (ctx->h_read)
+            HIP_TRY(hipHostFree(ctx->h_read));
+        ctx->h_read = nullptr;
+        ctx->h_read_n = 0;
+        HIP_TRY(hipHostMalloc((void **)&ctx->h_read, size, hipHostMallocDefault));
+        ctx->h_read_n = size;
+    }
+    // the body's row of the device states; without one (no update since it was created) the host's is current
+    const bool row = ctx->states_on_device && (size_t)body < ctx->d_states.n;
+    const ReadSources src{ pos ? b.dev.x : nullptr, prev ? b.dev.prev : nullptr, vel ? b.dev.v : nullptr, plane ? b.dev.plane : nullptr,
+                           shape_idx ? b.dev.idx : nullptr, contact ? b.dev.contact : nullptr,
+                           row ? ctx->d_states.p + body : nullptr, ctx->d_error.p };
+    ReadHeader *header = reinterpret_cast<ReadHeader *>(ctx->h_read);
+    const uint32_t *in = reinterpret_cast<const uint32_t *>(ctx->h_read + kHeader);
+    HIP_TRY(launch_readback(src, b.nv, header, const_cast<uint32_t *>(in), ctx->stream));
+    HIP_TRY(hipStreamSynchronize(ctx->stream));
+    if (int rc = CheckError(ctx, header->error))
         return rc;
-    if (shape_idx)
-        HIP_TRY(hipMemcpy(shape_idx, b.dev.idx, sizeof(int32_t) * nv, hipMemcpyDeviceToHost));
-    if (contact)
-        HIP_TRY(hipMemcpy(contact, b.dev.contact, sizeof(int32_t) * nv, hipMemcpyDeviceToHost));
+    auto take = [&](void *dst, size_t per_vertex) {
+        if (!dst)
+            return;
+        memcpy(dst, in, 4 * per_vertex * nv);
+        in += per_vertex * nv;
+    };
+    take(pos, 3);
+    take(prev, 3);
+    take(vel, 3);
+    take(plane, 4);
+    take(shape_idx, 1);
+    take(contact, 1);
+    if (row)
+        b.state = header->state;
     if (body_pos)
         memcpy(body_pos, b.state.pos, sizeof(b.state.pos));
     if (body_rot)

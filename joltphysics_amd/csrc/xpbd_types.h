@@ -143,6 +143,20 @@ struct BodyStateDev
     int32_t active;
 };
 
+// What a read-back packs for the host (xpbd_readback.hip): a null source is not wanted.
+struct ReadSources
+{
+    const float4 *x, *prev, *v, *plane;
+    const int32_t *idx, *contact;
+    const BodyStateDev *state;
+    const int32_t *error;
+};
+struct ReadHeader
+{
+    BodyStateDev state;
+    int32_t error;
+};
+
 // Convex hull data in device memory (a context-wide table, one entry per hull collider)
 struct HullDev
 {
