@@ -354,13 +354,11 @@ __device__ __forceinline__ void volume_adjoint(float4 *A, uint32_t k, uint32_t i
     // d4 = (x2 - x1) x (x3 - x1)
     g = quad_cross(x1x3, e4); h = quad_cross(e4, x1x2);
     b2 = b2 + g; b3 = b3 + h; b1 = b1 - g - h;
-    if (!(denom < 1.0e-12f))
-    {
-        cset(A, i1, k, b1);
-        cset(A, i2, k, b2);
-        cset(A, i3, k, b3);
-        cset(A, i4, k, b4);
-    }
+    const bool keep = denom < 1.0e-12f;
+    cset(A, i1, k, keep ? y1 : b1);
+    cset(A, i2, k, keep ? y2 : b2);
+    cset(A, i3, k, keep ? y3 : b3);
+    cset(A, i4, k, keep ? y4 : b4);
 }
 
 // Adjoint of an edge from delta and length before its projection (formulas above), component k of
@@ -383,11 +381,8 @@ __device__ __forceinline__ float edge_adjoint(float4 *A, uint32_t lane, uint32_t
     const float n = delta / length;
     const float nc = quad_dot(n, cbar);
     const float dbar = (c_length * cbar + (rest_length * nc) * n) / s;
-    if (acts)
-    {
-        cset(A, i0, k, a0 - dbar);
-        cset(A, i1, k, a1 + dbar);
-    }
+    cset(A, i0, k, acts ? a0 - dbar : a0);
+    cset(A, i1, k, acts ? a1 + dbar : a1);
     // correction = n c / s, alphabar += (cbar . correction) (-1 / (h^2 s))
     return acts ? (nc * c) * inv_s * (-inv_dt_sq * inv_s) : 0.0f;
 }
@@ -598,44 +593,49 @@ __device__ __forceinline__ void project_levels(const RolloutBodyDev &B, const St
 template <bool TAPE, bool BENDS>
 __device__ __forceinline__ void project_tasks(const RolloutBodyDev &B, float4 *X, float inv_dt_sq, uint32_t tid, float4 *tape)
 {
-    const uint32_t lane = tid & (kWave - 1u), quad = lane >> 2, c = (lane & 3u) < 2u ? (lane & 3u) : 2u;
+    const uint32_t lane = tid & (kWave - 1u), c = (lane & 3u) < 2u ? (lane & 3u) : 2u;
     const uint32_t stride = B.tape_stride;
     TaskStream<> tasks;
     tasks.begin(B.task_recs, B.task_desc, B.task_heads + (tid >> 6), lane);
     tasks.run(lane, [&](uint32_t d, const uint4 &r, NoAux::Value, uint32_t first) {
-        const uint32_t n = d & 127u, kind = (d >> 7) & 7u;
+        const uint32_t n = d & 127u;
         const uint32_t i0 = r.x & 0x3fffu, i1 = r.x >> 16, i2 = r.y & 0x3fffu, i3 = r.y >> 16;
         const float p0 = __uint_as_float(r.z), p1 = __uint_as_float(r.w);
-        if (kind == kTaskEdgeQuad)
+        // the tape entry of this lane's record; quads past the last repeat it, as they do the record
+        auto entry = [&] { return tape + (size_t)stride * (first + ((lane >> 2) < n ? lane >> 2 : n - 1u)); };
+        auto tape_positions = [&] {
+            if (TAPE && (lane & 3u) < 3u)
+                entry()[c] = make_float4(cget(X, i0, c), cget(X, i1, c), cget(X, i2, c), cget(X, i3, c));
+        };
+        if (opaque_kind(d) == kTaskEdgeQuad)
         {
-            if (quad < n)
-            {
-                float delta, length;
-                project_edge_quad(X, c, i0, i1, p0, p1, inv_dt_sq, delta, length);
-                if (TAPE)
-                    reinterpret_cast<float *>(tape + (size_t)stride * (first + quad))[lane & 3u] = (lane & 3u) == 3u ? length : delta;
-            }
-        }
-        else if (kind == kTaskVolumeQuad || (BENDS && kind == kTaskBendQuad))
-        {
-            if (quad < n)
-            {
-                if (TAPE && (lane & 3u) < 3u)
-                    tape[(size_t)stride * (first + quad) + c] = make_float4(cget(X, i0, c), cget(X, i1, c), cget(X, i2, c), cget(X, i3, c));
-                if (BENDS && kind == kTaskBendQuad)
-                    project_bend_quad(X, c, i0, i1, i2, i3, p0, p1, inv_dt_sq);
-                else
-                    project_volume_quad(X, c, i0, i1, i2, i3, p0, p1, inv_dt_sq);
-            }
-        }
-        else if (lane < n && i0 != i1)
-        {
+            float delta, length;
+            project_edge_quad(X, false, c, i0, i1, p0, p1, inv_dt_sq, delta, length);
             if (TAPE)
+                reinterpret_cast<float *>(entry())[lane & 3u] = (lane & 3u) == 3u ? length : delta;
+        }
+        if (opaque_kind(d) != kTaskEdgeQuad)
+        {
+            if (opaque_kind(d) == kTaskVolumeQuad)
             {
-                const V3 delta = xyz(X[i1]) - xyz(X[i0]);
-                tape[(size_t)stride * (first + lane)] = f4(delta, len_sq(delta));
+                tape_positions();
+                project_volume_quad(X, false, c, i0, i1, i2, i3, p0, p1, inv_dt_sq);
             }
-            project_lra(X, i0, i1, p0);
+            if (BENDS && opaque_kind(d) == kTaskBendQuad)
+            {
+                tape_positions();
+                project_bend_quad(X, false, c, i0, i1, i2, i3, p0, p1, inv_dt_sq);
+            }
+            if (opaque_kind(d) < kTaskVolumeQuad)
+                if (lane < n && i0 != i1)
+                {
+                    if (TAPE)
+                    {
+                        const V3 delta = xyz(X[i1]) - xyz(X[i0]);
+                        tape[(size_t)stride * (first + lane)] = f4(delta, len_sq(delta));
+                    }
+                    project_lra(X, i0, i1, p0);
+                }
         }
     });
 }
@@ -660,40 +660,36 @@ template <bool BENDS>
 __device__ __forceinline__ void reverse_tasks(const RolloutBodyDev &B, float4 *A, float *alpha_bar, float inv_dt_sq, uint32_t tid,
                                               const float4 *tape)
 {
-    const uint32_t lane = tid & (kWave - 1u), quad = lane >> 2, c = (lane & 3u) < 2u ? (lane & 3u) : 2u;
+    const uint32_t lane = tid & (kWave - 1u), c = (lane & 3u) < 2u ? (lane & 3u) : 2u;
     const TapeAux aux{ tape, B.tape_stride };
     TaskStream<true, TapeAux> tasks;
     tasks.begin(B.task_recs, B.task_desc, B.task_heads + (tid >> 6), lane, aux);
     tasks.run(lane, [&](uint32_t d, const uint4 &r, const RecordVec &tv, uint32_t first) {
-        const uint32_t n = d & 127u, kind = (d >> 7) & 7u;
+        const uint32_t n = d & 127u;
         const uint32_t i0 = r.x & 0x3fffu, i1 = r.x >> 16, i2 = r.y & 0x3fffu, i3 = r.y >> 16;
         const float p0 = __uint_as_float(r.z), p1 = __uint_as_float(r.w);
         const float4 t = make_float4(__uint_as_float(tv.x), __uint_as_float(tv.y), __uint_as_float(tv.z), __uint_as_float(tv.w));
-        if (kind == kTaskEdgeQuad)
+        // quads past the last record repeat it and store the same values
+        if (opaque_kind(d) == kTaskEdgeQuad)
         {
-            if (quad < n)
-            {
-                const float delta = c == 0 ? t.x : c == 1 ? t.y : t.z;
-                const float alpha = edge_adjoint(A, lane, c, i0, i1, delta, t.w, p0, p1, inv_dt_sq);
-                if ((lane & 3u) == 0u)
-                    alpha_bar[r.y] += alpha;
-            }
+            const float delta = c == 0 ? t.x : c == 1 ? t.y : t.z;
+            const float alpha = edge_adjoint(A, lane, c, i0, i1, delta, t.w, p0, p1, inv_dt_sq);
+            if ((lane & 3u) == 0u)
+                alpha_bar[r.y] += alpha;
         }
-        else if (kind == kTaskVolumeQuad)
+        if (opaque_kind(d) != kTaskEdgeQuad)
         {
-            if (quad < n)
+            if (opaque_kind(d) == kTaskVolumeQuad)
                 volume_adjoint(A, c, i0, i1, i2, i3, t, p0, p1, inv_dt_sq);
-        }
-        else if (BENDS && kind == kTaskBendQuad)
-        {
-            if (quad < n)
+            if (BENDS && opaque_kind(d) == kTaskBendQuad)
             {
-                const float4 *q = tape + (size_t)B.tape_stride * (first + quad);
+                const float4 *q = tape + (size_t)B.tape_stride * (first + ((lane >> 2) < n ? lane >> 2 : n - 1u));
                 bend_adjoint(A, lane, i0, i1, i2, i3, q[0], q[1], q[2], p0, p1, inv_dt_sq);
             }
+            if (opaque_kind(d) < kTaskVolumeQuad)
+                if (lane < n && i0 != i1)
+                    lra_adjoint(A, i0, i1, t, p0);
         }
-        else if (lane < n && i0 != i1)
-            lra_adjoint(A, i0, i1, t, p0);
     }, aux);
     __syncthreads();
 }

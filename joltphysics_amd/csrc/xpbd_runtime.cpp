@@ -496,7 +496,7 @@ struct GroupLevels
 struct TaskProgram
 {
     std::vector<uint4> recs;        // per wavefront, in task order; one record behind the last
-    std::vector<uint32_t> desc;     // per wavefront, kDescPad zero descriptors before and behind each list
+    std::vector<uint32_t> desc;     // per wavefront, kTaskDescPad zero descriptors before and behind each list
     std::vector<uint4> heads;       // per wavefront {first descriptor, tasks, first record, trailing barriers}, then
                                     // one with the end of the records
     double ns = 0.0;                // estimated duration of one run
@@ -504,8 +504,6 @@ struct TaskProgram
 
 struct TaskBuilder
 {
-    // a step fetches descriptors six tasks ahead and runs three tasks at a time
-    static constexpr uint32_t kDescPad = 12;
     // Instructions of one projection by type (volume, bend, edge, LRA), on one lane and on four.
     // A lone wavefront issues one instruction in about 5 cycles and a SIMD one in 4, so a level
     // takes its longest task or a quarter of all its tasks, whichever is more: narrow levels
@@ -606,11 +604,11 @@ struct TaskBuilder
     {
         for (uint32_t w = 0; w < waves; ++w)
         {
-            out.desc.insert(out.desc.end(), kDescPad, 0u);
+            out.desc.insert(out.desc.end(), kTaskDescPad, 0u);
             out.heads.push_back(make_uint4((uint32_t)out.desc.size(), (uint32_t)wdesc[w].size(), (uint32_t)out.recs.size(), pending[w]));
             out.recs.insert(out.recs.end(), wrecs[w].begin(), wrecs[w].end());
             out.desc.insert(out.desc.end(), wdesc[w].begin(), wdesc[w].end());
-            out.desc.insert(out.desc.end(), kDescPad, 0u);
+            out.desc.insert(out.desc.end(), kTaskDescPad, 0u);
         }
         out.heads.push_back(make_uint4(0u, 0u, (uint32_t)out.recs.size(), 0u));
         out.recs.push_back(make_uint4(0u, 0u, 0u, 0u));     // read, not used, behind a task's records

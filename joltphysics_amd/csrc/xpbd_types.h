@@ -23,6 +23,9 @@ constexpr uint32_t kMaxWindowVertices = 1u << 14;
 
 // Wavefronts of a workgroup that runs a streamed body or a team member (1024 threads)
 constexpr uint32_t kStreamedWaves = 16;
+// Task programs: zero descriptors before and behind each wavefront's list (a step fetches them six
+// tasks ahead, and tasks run three at a time)
+constexpr uint32_t kTaskDescPad = 12;
 
 // A window is a set of vertices held in LDS while a run of levels executes on
 // it.  Resident bodies keep all their vertices in LDS for the whole launch and
