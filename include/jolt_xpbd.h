@@ -403,8 +403,8 @@ int xpbd_update(xpbd_context *ctx, float dt, int32_t collision_steps, int32_t fr
  * groups over its job threads), the non-parallel group follows on one of them, and the
  * per-vertex phases are split.  Results are bit-identical to the one-workgroup path.
  * Bodies with rods or pressure, and contexts with dynamic or sensor colliders, keep the
- * one-workgroup path.  Default 3, or 2 while a workgroup per window of all such bodies fits the
- * card at once; 0 never forms teams.  No reference counterpart (a scheduling choice).
+ * one-workgroup path.  Default 3; 0 never forms teams.  No reference counterpart (a
+ * scheduling choice).
  */
 int xpbd_context_set_team_min_windows(xpbd_context *ctx, uint32_t windows);
 /* Workgroups per team at least (0, the default: one per parallel-group window, two for a body

@@ -772,8 +772,8 @@ __device__ __forceinline__ void run_levels_global(const uint4 *recs, const uint3
 // loads in program order, so a step waits for no load issued in the last two steps; the level
 // offsets of run_program_global are scalar loads whose latency, like its exec-masked kinds, is
 // paid in every level.  An empty level costs 80 ns here and 145 to 229 ns there; a level of a
-// 90 x 90 cloth (31 bends, 37 edges) 745 ns against 1,010, one of a 16-cell cube 485 against 590,
-// one of the coloured cloth (512 bends, 600 edges) 2,200 against 3,500 (512 threads).
+// 90 x 90 cloth (31 bends, 37 edges) 663 ns against 1,024, one of a 16-cell cube 425 against 562,
+// one of the coloured cloth (512 bends, 600 edges) 2,135 against 3,450 (512 threads).
 enum TaskKind : uint32_t { kTaskVolume = 0, kTaskBend = 1, kTaskEdge = 2, kTaskLRA = 3, kTaskVolumeQuad = 4, kTaskBendQuad = 5, kTaskEdgeQuad = 6 };
 constexpr uint32_t kTaskQuadBit = 4u << 7;
 

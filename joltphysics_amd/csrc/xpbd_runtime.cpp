@@ -265,7 +265,6 @@ struct xpbd_context
     std::vector<uint32_t> streamed;
     // large streamed bodies run by teams of workgroups (xpbd_team.hip)
     uint32_t team_min_windows = 3;  // a streamed body with this many parallel-group windows gets a team (0: never)
-    bool team_min_windows_set = false;      // not set: two-window bodies get one too while there is room (BuildTeams)
     uint32_t team_size = 0;         // workgroups per team at least (0: one per parallel-group window)
     std::vector<TeamDev> teams;
     std::vector<uint2> team_blocks; // per workgroup of the team launch: team, member
@@ -1394,11 +1393,7 @@ double StreamedMicroseconds(const Body &b)
 // when it asks for the coloured non-parallel group.  One member per window (the
 // windows' levels then run concurrently), at most kMaxTeamBlocks workgroups in all, so
 // that every member of every team holds a CU at once; each member takes a contiguous
-// run of windows of about equal cost.  While team_min_windows is left alone a body of two
-// windows gets a team as well, if all of them fit beside the larger bodies' teams with a
-// workgroup per window: a 127 x 113 cloth (windows of 233 and 287 levels, 769 levels behind
-// them) 9.6 -> 7.4 ms per frame for 2 CUs instead of one.  With more such bodies than that the
-// CUs are better spent on a body each (9.6 CU-milliseconds against 14.8).
+// run of windows of about equal cost.
 constexpr uint32_t kMaxTeamBlocks = 224;
 constexpr uint32_t kMaxTeamSize = 224;
 
@@ -1407,45 +1402,24 @@ int BuildTeams(xpbd_context *ctx)
     ctx->teams.clear();
     ctx->team_blocks.clear();
     std::vector<uint32_t> keep, members;
-    auto is_eligible = [&](const Body &b) {
-        const xpbd_settings &st = *b.settings;
-        return !st.dev.resident && st.rods.empty() && !(b.dev.pressure > 0.0f && st.num_faces > 0) && ctx->num_dynamic == 0
-               && ctx->num_sensors == 0;
-    };
-    // one member per window; a coloured body's colour passes take twice that by default
-    auto team_members = [&](const Body &b) {
-        const uint32_t windows = b.settings->dev.num_par_windows;
-        const uint32_t want = ctx->team_size ? ctx->team_size : (b.tail_mode == XPBD_TAIL_COLOURED ? 2u : 1u) * windows;
-        return std::max(1u, std::min(std::max(windows, want), kMaxTeamSize));
-    };
-    uint32_t min_windows = ctx->team_min_windows;
-    if (!ctx->team_min_windows_set)
-    {
-        uint32_t wanted = 0;
-        for (uint32_t i : ctx->streamed)
-        {
-            const Body &b = *ctx->bodies[i];
-            if (is_eligible(b) && (b.tail_mode == XPBD_TAIL_COLOURED || b.settings->dev.num_par_windows >= 2))
-                wanted += team_members(b);
-        }
-        if (wanted <= kMaxTeamBlocks)
-            min_windows = 2;
-    }
     for (uint32_t i : ctx->streamed)
     {
         const Body &b = *ctx->bodies[i];
         const xpbd_settings &st = *b.settings;
-        const bool eligible = is_eligible(b);
+        const bool eligible = !st.dev.resident && st.rods.empty() && !(b.dev.pressure > 0.0f && st.num_faces > 0)
+                              && ctx->num_dynamic == 0 && ctx->num_sensors == 0;
         const bool coloured = b.tail_mode == XPBD_TAIL_COLOURED;
         if (coloured && !(eligible && st.colourable))
             return Fail(XPBD_E_UNSUPPORTED, "body " + std::to_string(i) + ": the coloured non-parallel group needs a streamed body "
                                             "(over 8192 vertices) without rods, pressure, skinned constraints in that group, "
                                             "dynamic or sensor colliders");
-        if (eligible && (coloured || (min_windows > 0 && st.dev.num_par_windows >= min_windows)))
+        if (eligible && (coloured || (ctx->team_min_windows > 0 && st.dev.num_par_windows >= ctx->team_min_windows)))
         {
             ctx->teams.push_back(TeamDev{});
             ctx->teams.back().body = i;
-            members.push_back(team_members(b));
+            // one member per window; a coloured body's colour passes take twice that by default
+            const uint32_t want = ctx->team_size ? ctx->team_size : (coloured ? 2u : 1u) * st.dev.num_par_windows;
+            members.push_back(std::max(1u, std::min(std::max(st.dev.num_par_windows, want), kMaxTeamSize)));
         }
         else
             keep.push_back(i);
@@ -2024,10 +1998,9 @@ int xpbd_context_set_team_min_windows(xpbd_context *ctx, uint32_t windows)
 {
     if (!ctx)
         return Fail(XPBD_E_INVALID, "null context");
-    if (ctx->team_min_windows != windows || !ctx->team_min_windows_set)
+    if (ctx->team_min_windows != windows)
     {
         ctx->team_min_windows = windows;
-        ctx->team_min_windows_set = true;
         ctx->layout_dirty = true;
     }
     return XPBD_OK;

@@ -32,10 +32,9 @@ namespace xpbd {
 
 constexpr int kTeamBlock = 1024;
 constexpr int kTeamWaves = kTeamBlock / kWave;
-// error bit of a barrier that waited too long (the realtime counter runs at 100 MHz: 10 s, so that
-// a member kept from its CU by the long launches of other streams is waited for)
+// error bit of a barrier that waited too long (the realtime counter runs at 100 MHz: 2 s)
 constexpr int32_t kErrTeamTimeout = 4;
-constexpr uint64_t kTeamSpinTicks = 1000000000ull;
+constexpr uint64_t kTeamSpinTicks = 200000000ull;
 
 struct TeamLds
 {
