@@ -77,6 +77,14 @@ def float_equal(a, b):
     return a.shape == b.shape and bool(np.all(a == b))
 
 
+def require_reference(variant="nofma"):
+    """Skips the calling test where the reference library is not built (it needs the reference sources)."""
+    import pytest
+    from oracle import have_reference
+    if not have_reference(variant):
+        pytest.skip("reference library not built (needs the reference sources)")
+
+
 def reference_run(scene, frames_to_keep, variant="nofma", num_threads=0, record_contacts=False, settings=None,
                   bodies=None):
     """Builds settings with the reference's own code (unless `settings` are given: one per
@@ -86,6 +94,7 @@ def reference_run(scene, frames_to_keep, variant="nofma", num_threads=0, record_
 
     Returns (settings_list, collider_bounds[n,6], {frame: [read(body)...]}), the reads in
     the order of `bodies`."""
+    require_reference(variant)
     from oracle import JoltReference, JoltWorld
     ref = JoltReference(variant)
     if settings is None:
@@ -143,6 +152,7 @@ def reference_custom_run(scene, frames_to_keep, variant="nofma", contact_setting
     colliders' velocities changed by UpdateRigidBodyVelocities.  Sets each collider's device
     parameters and initial motion from the reference.  Returns (settings, bounds,
     {frame: [read(body)]}, {frame: [(linear, angular) velocity of each collider]})."""
+    require_reference(variant)
     from oracle import JoltReference, JoltWorld
     assert len(scene.bodies) == 1 and scene.collision_steps == 1
     ref = JoltReference(variant)

@@ -10,7 +10,7 @@ import numpy as np
 import pytest
 
 import scene_zoo
-from helpers import float_equal, max_abs, recoloured_settings, reference_run, run_gpu
+from helpers import float_equal, max_abs, recoloured_settings, reference_run, require_reference, run_gpu
 
 pytestmark = pytest.mark.gpu
 
@@ -20,6 +20,7 @@ SCENES = ("tetcube_plane_box", "pressure_sphere", "lra_cloth", "batched", "cloth
 
 @pytest.mark.parametrize("name", SCENES)
 def test_coloured_schedule_equals_reference_on_recoloured_settings(name):
+    require_reference()
     sc = scene_zoo.ALL[name]()
     frames = tuple(sorted({1, 2, min(sc.frames, 6)}))
     from oracle import JoltReference

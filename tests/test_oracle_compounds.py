@@ -11,11 +11,13 @@ import numpy as np
 import pytest
 
 import scene_zoo
+from helpers import require_reference
 from joltphysics_amd.records import OP_CULL, OP_OFFSET, OP_ROTATE, OP_TRANSLATE, SHAPE_BOX, SHAPE_SPHERE, SHAPE_TAPERED_CAPSULE, \
     ShapeSpec
 
 
 def _worlds(colliders):
+    require_reference()
     from oracle import JoltReference, JoltWorld, Restatement
     w = JoltWorld(JoltReference("nofma"), (0.0, 0.0, -9.81))
     ids = [w.add_collider(c) for c in colliders]
