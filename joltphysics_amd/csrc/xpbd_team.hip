@@ -14,7 +14,8 @@
 // Members hand positions to each other through global memory across a team
 // barrier: every wavefront's stores complete, one thread releases at agent scope
 // (the members may sit on different XCDs, whose L2 caches are not coherent with each
-// other) and counts itself in, waits for the team's count, and acquires at agent scope.
+// other), waits for the write-back and counts itself in, waits for the team's count, and
+// acquires at agent scope.
 // Every wait is bounded: a barrier that waits longer than kTeamSpinTicks sets an
 // error bit, and from then on no barrier of the launch waits, so the launch always
 // drains.
@@ -52,6 +53,13 @@ __host__ __device__ inline TeamLds team_lds_layout(uint32_t window_capacity, uin
     return l;
 }
 
+// The L2 write-back or invalidation that a fence issued has completed.  The compiler does not
+// count these among the pending memory operations: after a wait that leaves none pending it
+// removes the wait that belongs to the fence, and the members would be counted in while their
+// stores are still on their way out of the XCD's L2 (a long way where other launches have filled it
+// with dirty lines).
+__device__ __forceinline__ void wait_cache_operation() { asm volatile("s_waitcnt vmcnt(0)" ::: "memory"); }
+
 // Team barrier.  `target` = team size x number of this barrier in the launch.
 __device__ __forceinline__ void team_barrier(uint32_t *counter, uint32_t target, int32_t *error_flag)
 {
@@ -60,6 +68,7 @@ __device__ __forceinline__ void team_barrier(uint32_t *counter, uint32_t target,
     if (threadIdx.x == 0)
     {
         __builtin_amdgcn_fence(__ATOMIC_RELEASE, "agent");
+        wait_cache_operation();
         __hip_atomic_fetch_add(counter, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
         const uint64_t t0 = __builtin_amdgcn_s_memrealtime();
         while ((int32_t)(__hip_atomic_load(counter, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) - target) < 0)
@@ -74,6 +83,7 @@ __device__ __forceinline__ void team_barrier(uint32_t *counter, uint32_t target,
             }
         }
         __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "agent");
+        wait_cache_operation();
     }
     __syncthreads();
 }
