@@ -573,10 +573,12 @@ int xpbd_profile_read(xpbd_context *ctx, int32_t *num_launches, double *total_ms
  * is the body-local vertex positions after `frames` frames.
  *
  * The backward pass is a hand-written adjoint: (x, v) checkpoints every
- * checkpoint_interval frames, each segment recomputed forward, then every
- * substep re-run with its pre-projection positions recorded and reversed level
- * by level in reverse order.  It returns d(loss)/d(compliance) and
- * d(loss)/d(initial velocity) given d(loss)/d(final positions).
+ * checkpoint_interval frames, each segment recomputed forward with what every
+ * projection's adjoint needs recorded (a tape of the whole segment while the
+ * segment tapes of the context's rollouts take at most 8 GiB and an eighth of the
+ * free device memory; else of one substep, which is run again for it), then
+ * reversed substep by substep, level by level.  It returns d(loss)/d(compliance)
+ * and d(loss)/d(initial velocity) given d(loss)/d(final positions).
  *
  * All array arguments are device pointers; `stream` is the hipStream_t the
  * work is ordered on (NULL: the default stream, as torch's default stream is;

@@ -251,6 +251,8 @@ struct xpbd_context
     // pinned host memory a read-back packs a body into, at most twice what the largest read needed
     unsigned char *h_read = nullptr;
     size_t h_read_n = 0;
+    // bytes of whole-segment tapes of the context's rollouts, each of which holds the count too
+    std::shared_ptr<size_t> tape_bytes = std::make_shared<size_t>(0);
     float gravity[3] = { 0.0f, -9.81f, 0.0f };       // PhysicsSystem.h:392 default
     bool profiling = false;
     std::vector<std::pair<hipEvent_t, hipEvent_t>> events;
@@ -3282,19 +3284,25 @@ struct xpbd_rollout
     RolloutDev dev{};
     uint32_t total_nv = 0, total_ne = 0;
     uint32_t lds_f32 = 0, lds_f64 = 0, lds_bwd = 0;
+    std::shared_ptr<size_t> tape_bytes;     // the context's
+    size_t segment_tape = 0;    // bytes of a whole segment's tape, 0: of one sub-step's only
     bool bends = false;         // some body has dihedral bends
     bool has_forward = false;
 
     ~xpbd_rollout()
     {
+        if (tape_bytes)
+            *tape_bytes -= segment_tape;
         for (xpbd_settings *s : settings)
             xpbd_settings_release(s);
     }
 };
 
 namespace {
-// Largest segment tape of a rollout (the GPU has 288 GB)
+// Largest segment tapes of a context's rollouts together (the GPU has 288 GB), and the share of the
+// memory free when a rollout is created that its tape may take.
 constexpr size_t kTapeBytes = (size_t)8 << 30;
+constexpr size_t kTapeFreeShare = 8;
 
 // The caller's stream as given: NULL is the default (null) stream, as in torch.
 hipStream_t StreamOf(xpbd_rollout *, void *stream) { return (hipStream_t)stream; }
@@ -3433,12 +3441,28 @@ int xpbd_rollout_create(xpbd_context *ctx, const xpbd_rollout_desc *d, xpbd_roll
     HIP_TRY(r->seg_x.alloc((seg_sub + 1) * nv)); HIP_TRY(r->seg_v.alloc(seg_sub * nv));
     HIP_TRY(r->vel.alloc(nv)); HIP_TRY(r->prev.alloc(nv));
     HIP_TRY(r->vel64.alloc(4 * nv)); HIP_TRY(r->prev64.alloc(4 * nv));
-    // The tape of a whole segment when it fits the budget (the adjoint then needs no second
-    // forward sweep of every sub-step), else of one sub-step.
-    const uint32_t tape_subs = std::min<size_t>(seg_sub, (size_t)d->frames * d->num_iterations) * tape * sizeof(float4) <= kTapeBytes
-                                   ? (uint32_t)std::min<size_t>(seg_sub, (size_t)d->frames * d->num_iterations) : 1u;
-    HIP_TRY(r->tape.alloc(tape * tape_subs));
     HIP_TRY(r->adj_x.alloc(nv)); HIP_TRY(r->adj_v.alloc(nv));
+    // The tape of a whole segment when it fits the budget (the adjoint then needs no second
+    // forward sweep of every sub-step: 64 cloths of 64 x 64 in segments of 50 sub-steps, 0.8 GB,
+    // 100 ms instead of 127 for a forward and an adjoint), else of one sub-step.  A rollout that
+    // only runs forward takes it as well, since no later call may allocate, so it never takes more
+    // than a share of what is free.
+    uint32_t tape_subs = (uint32_t)std::min<size_t>(seg_sub, (size_t)d->frames * d->num_iterations);
+    const size_t segment = tape * tape_subs * sizeof(float4);
+    size_t free_bytes = 0, total_bytes = 0;
+    HIP_TRY(hipMemGetInfo(&free_bytes, &total_bytes));
+    if (tape_subs > 1 && (*ctx->tape_bytes + segment > kTapeBytes || segment > free_bytes / kTapeFreeShare))
+        tape_subs = 1;
+    if (tape_subs > 1 && r->tape.alloc(tape * tape_subs) != hipSuccess)
+    {
+        (void)hipGetLastError();        // what is free is in pieces: one sub-step's tape will do
+        tape_subs = 1;
+    }
+    if (tape_subs == 1)
+        HIP_TRY(r->tape.alloc(tape));
+    r->tape_bytes = ctx->tape_bytes;
+    r->segment_tape = tape_subs > 1 ? segment : 0;
+    *r->tape_bytes += r->segment_tape;
     RolloutDev &R = r->dev;
     R.bodies = r->bodies.p;
     R.num_bodies = d->num_bodies;
