@@ -248,7 +248,7 @@ struct xpbd_context
     DevBuf<DynStateDev> d_dyn;      // bodies x num_dynamic
     uint32_t dyn_stride = 0;        // num_dynamic the rows of d_dyn are laid out for
     DevBuf<int32_t> d_error;
-    // pinned host memory a read-back packs a body into, at most twice what the largest read needed
+    // pinned host memory a read-back packs a body into
     unsigned char *h_read = nullptr;
     size_t h_read_n = 0;
     // bytes of whole-segment tapes of the context's rollouts, each of which holds the count too
@@ -1508,8 +1508,31 @@ int BuildTeams(xpbd_context *ctx)
     return XPBD_OK;
 }
 
+// Read-back: a header, then the requested arrays (at most all of them: 15 words a vertex)
+constexpr size_t kReadHeader = (sizeof(ReadHeader) + 255) / 256 * 256;
+constexpr size_t kReadVertex = 15 * 4;
+
+int ReserveRead(xpbd_context *ctx, size_t bytes)
+{
+    if (ctx->h_read_n >= bytes)
+        return XPBD_OK;
+    if (ctx->h_read)
+        HIP_TRY(hipHostFree(ctx->h_read));
+    ctx->h_read = nullptr;
+    ctx->h_read_n = 0;
+    HIP_TRY(hipHostMalloc((void **)&ctx->h_read, bytes, hipHostMallocDefault));
+    ctx->h_read_n = bytes;
+    return XPBD_OK;
+}
+
 int BuildLayout(xpbd_context *ctx)
 {
+    // once for the largest body here, so that no read has to pin memory
+    size_t largest = 0;
+    for (const auto &b : ctx->bodies)
+        largest = std::max<size_t>(largest, b->nv);
+    if (int rc = ReserveRead(ctx, kReadHeader + kReadVertex * largest))
+        return rc;
     const uint32_t nc = (uint32_t)ctx->colliders.size();
     // A body joins the bundles when its identity program exists and its positions
     // fit in one workgroup's LDS: 12 B per vertex when all its vertices share one
@@ -2758,25 +2781,16 @@ int xpbd_body_read(xpbd_context *ctx, int32_t body, float *pos, float *prev, flo
     Body &b = *ctx->bodies[body];
     const size_t nv = b.nv;
     const size_t words = nv * ((pos ? 3 : 0) + (prev ? 3 : 0) + (vel ? 3 : 0) + (plane ? 4 : 0) + (shape_idx ? 1 : 0) + (contact ? 1 : 0));
-    constexpr size_t kHeader = (sizeof(ReadHeader) + 255) / 256 * 256;
-    const size_t need = kHeader + 4 * words;
-    if (ctx->h_read_n < need)
-    {
-        const size_t size = std::max(need, 2 * ctx->h_read_n);
-        if (ctx->h_read)
-            HIP_TRY(hipHostFree(ctx->h_read));
-        ctx->h_read = nullptr;
-        ctx->h_read_n = 0;
-        HIP_TRY(hipHostMalloc((void **)&ctx->h_read, size, hipHostMallocDefault));
-        ctx->h_read_n = size;
-    }
+    // before the first update of a layout there may be no buffer, or one for smaller bodies
+    if (int rc = ReserveRead(ctx, kReadHeader + 4 * words))
+        return rc;
     // the body's row of the device states; without one (no update since it was created) the host's is current
     const bool row = ctx->states_on_device && (size_t)body < ctx->d_states.n;
     const ReadSources src{ pos ? b.dev.x : nullptr, prev ? b.dev.prev : nullptr, vel ? b.dev.v : nullptr, plane ? b.dev.plane : nullptr,
                            shape_idx ? b.dev.idx : nullptr, contact ? b.dev.contact : nullptr,
                            row ? ctx->d_states.p + body : nullptr, ctx->d_error.p };
     ReadHeader *header = reinterpret_cast<ReadHeader *>(ctx->h_read);
-    const uint32_t *in = reinterpret_cast<const uint32_t *>(ctx->h_read + kHeader);
+    const uint32_t *in = reinterpret_cast<const uint32_t *>(ctx->h_read + kReadHeader);
     HIP_TRY(launch_readback(src, b.nv, header, const_cast<uint32_t *>(in), ctx->stream));
     HIP_TRY(hipStreamSynchronize(ctx->stream));
     if (int rc = CheckError(ctx, header->error))
