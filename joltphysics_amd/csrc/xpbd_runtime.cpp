@@ -1568,32 +1568,48 @@ int BuildLayout(xpbd_context *ctx)
             return mass_bits(a) < mass_bits(b);
         return A.settings->host_level_begin.size() > B.settings->host_level_begin.size();
     });
-    std::vector<std::unique_ptr<BundleHost>> bundles;
-    // Bodies share a workgroup only when there are more of them than the chip holds workgroups
-    // (two per CU): merged levels are wider and take longer, so a small scene spreads its bodies
-    // over the CUs.
-    size_t all_lds = 0;
-    for (uint32_t bi : resident)
-        all_lds += bundle_lds_bytes(ctx->bodies[bi]->nv, 1, uniform_of(bi));
-    const uint32_t pack_lds = (uint32_t)std::min<size_t>(kBundleClasses[0].lds, all_lds / kResidentWorkgroups);
-    for (uint32_t bi : resident)
-    {
-        const Body &b = *ctx->bodies[bi];
-        BundleHost *cur = bundles.empty() ? nullptr : bundles.back().get();
-        const bool same_class = cur && uniform_of(cur->bodies[0]) == uniform_of(bi)
-                                && (!uniform_of(bi) || mass_bits(cur->bodies[0]) == mass_bits(bi))
-                                && ctx->bodies[cur->bodies[0]]->dev.iterations == b.dev.iterations;
-        const bool fits = same_class && cur->bodies.size() < kBundleMaxBodies
-                          && bundle_lds_bytes(cur->nv + b.nv, (uint32_t)cur->bodies.size() + 1u, uniform_of(bi)) <= pack_lds;
-        if (!fits)
+    // Greedy packing in that order; none: a bundle of its own for every body
+    auto pack = [&](uint32_t cap, std::vector<std::vector<uint32_t>> &out) {
+        out.clear();
+        uint32_t nv = 0;
+        size_t slots = 0;
+        for (uint32_t bi : resident)
         {
-            bundles.emplace_back(new BundleHost);
-            cur = bundles.back().get();
-            cur->uniform = uniform_of(bi);
-            cur->inv_mass = b.settings->inv_mass;
+            const Body &b = *ctx->bodies[bi];
+            const uint32_t first = out.empty() ? 0u : out.back()[0];
+            const bool same_class = !out.empty() && uniform_of(first) == uniform_of(bi)
+                                    && (!uniform_of(bi) || mass_bits(first) == mass_bits(bi))
+                                    && ctx->bodies[first]->dev.iterations == b.dev.iterations;
+            if (!(same_class && out.back().size() < kBundleMaxBodies
+                  && bundle_lds_bytes(nv + b.nv, (uint32_t)out.back().size() + 1u, uniform_of(bi)) <= cap))
+            {
+                out.emplace_back();
+                nv = 0;
+                // a workgroup of the larger class takes a CU for itself
+                slots += bundle_lds_bytes(b.nv, 1, uniform_of(bi)) <= kBundleClasses[0].lds ? 1u : 2u;
+            }
+            out.back().push_back(bi);
+            nv += b.nv;
         }
-        cur->bodies.push_back(bi);
-        cur->nv += b.nv;
+        return slots;
+    };
+    // Merged levels are wider and take longer, but a workgroup that waits for another to end takes
+    // twice as long: bodies share workgroups only as tightly as it takes for the chip to run all of
+    // them at once (the least multiple of 1 KB that does it), and up to the smaller class where nothing
+    // does.  1,000 cloths of 32 x 32: 2.50 ms per frame on a workgroup each, 1.83 packed to 80 KB, 1.41 in pairs.
+    std::vector<std::vector<uint32_t>> packed;
+    for (uint32_t cap = 0; pack(cap, packed) > kResidentWorkgroups && cap < kBundleClasses[0].lds;)
+        cap += 1024u;
+    std::vector<std::unique_ptr<BundleHost>> bundles;
+    for (std::vector<uint32_t> &members : packed)
+    {
+        bundles.emplace_back(new BundleHost);
+        BundleHost &bh = *bundles.back();
+        bh.uniform = uniform_of(members[0]);
+        bh.inv_mass = ctx->bodies[members[0]]->settings->inv_mass;
+        for (uint32_t bi : members)
+            bh.nv += ctx->bodies[bi]->nv;
+        bh.bodies = std::move(members);
     }
 
     // Programs and launch classes: a bundle takes the smallest class its positions fit.
