@@ -763,7 +763,7 @@ __global__ __launch_bounds__(BLOCK) void rollout_forward_kernel(RolloutDev R, co
 // checkpoint keeping every sub-step's start state and, when it fits (R.tape_subs), every
 // sub-step's tape; then reverse it sub-step by sub-step.  A tape of one sub-step is filled by
 // running the sub-step again before its adjoint.  Measured on 64 cloths of 64 x 64 (60 frames x 5
-// iterations), forward and adjoint: 229 -> 114 ms; before, every sub-step ran a second forward
+// iterations), forward and adjoint: 229 -> 100 ms; before, every sub-step ran a second forward
 // sweep for its tape, whose loads stood exposed in every reverse level.
 template <int BLOCK, bool BENDS>
 __global__ __launch_bounds__(BLOCK) void rollout_backward_kernel(RolloutDev R, const float *__restrict__ grad_positions,

@@ -31,6 +31,7 @@ def _run(settings, sizes, iterations=2):
         ctx.update(1 / 60, 1, 2)
         places = [ctx.placement(i) for i in ids]
         assert all(p[0] == "bundle" for p in places)
+        _run.threads = {p[1] for p in places}
         return len({p[2] for p in places}), [ctx.read(ids[k])["pos"] for k in range(0, len(ids), 37)]
     finally:
         ctx.close()
@@ -53,3 +54,12 @@ def test_workgroups_and_results(settings, sizes):
         if key not in alone:
             alone[key] = _run(settings, [sizes[k]], 2 + key[1])[1][0]
         assert np.array_equal(g, alone[key]), f"body {k}"
+
+
+@pytest.mark.parametrize("side, count, threads", [(17, 1, 512), (17, 256, 512), (31, 1, 1024), (31, 256, 1024), (31, 257, 512)])
+def test_threads(settings, side, count, threads):
+    """Bodies of more than 512 vertices take 1024 threads while every workgroup has a CU to itself."""
+    workgroups, got = _run(settings, [side] * count)
+    assert workgroups == count and _run.threads == {threads}
+    want = _run(settings, [side])[1][0]
+    assert all(np.array_equal(g, want) for k, g in zip(range(0, count, 37), got) if k % 7 != 3)
