@@ -1612,13 +1612,16 @@ int BuildLayout(xpbd_context *ctx)
         bh.bodies = std::move(members);
     }
 
-    // Programs and launch classes: a bundle takes the smaller class if its positions fit, unless it has
-    // more vertices than that class has threads and every workgroup of the update has a CU to itself.
-    // Twice the wavefronts then halve the per-vertex phases and the wide levels: under the coloured
+    // Programs and launch classes: a bundle takes the smaller class if its positions fit, unless every
+    // workgroup of the update has a CU to itself and some bundle has more vertices than that class has
+    // threads.  Twice the wavefronts then halve its per-vertex phases and wide levels: under the coloured
     // schedule a 72 x 72 cloth 0.90 -> 0.75 ms, a 16-cell cube 1.10 -> 0.98, a 40 x 40 cloth on six hulls
-    // 0.82 -> 0.63; exact 4.48 -> 4.42, 4.11 -> 4.07, 3.18 -> 3.01.  Up to 512 vertices they cost a
-    // barrier's width, 1 % on a 17 x 9 cloth.
-    const bool own_cu = bundles.size() + ctx->streamed.size() + ctx->team_blocks.size() <= kResidentWorkgroups / 2u;
+    // 0.82 -> 0.63; exact 4.48 -> 4.42, 4.11 -> 4.07, 3.18 -> 3.01.  Up to 512 vertices they only make
+    // barriers wider, 1 % on a 17 x 9 cloth; beside a larger bundle such a body waits anyway, and one launch
+    // instead of two saves the streams' fork (12 us on 48 uneven bodies).
+    bool wide = bundles.size() + ctx->streamed.size() + ctx->team_blocks.size() <= kResidentWorkgroups / 2u;
+    if (wide)
+        wide = std::any_of(bundles.begin(), bundles.end(), [](const auto &bh) { return bh->nv > kBundleClasses[0].block; });
     struct Plan
     {
         std::vector<uint32_t> voffs;
@@ -1657,7 +1660,7 @@ int BuildLayout(xpbd_context *ctx)
         const uint32_t lds = bundle_lds_bytes(voff, nb, bh.uniform);
         if (lds > kMaxLdsBytes)
             return Fail(XPBD_E_CAPACITY, "bundle needs more LDS than a workgroup has");
-        P.cls = lds <= kBundleClasses[0].lds && !(own_cu && voff > kBundleClasses[0].block) ? 0 : 1;
+        P.cls = lds <= kBundleClasses[0].lds && !wide ? 0 : 1;
         // workgroups that share a CU share its four SIMDs
         const double simds = P.cls == 0 && bundles.size() > kResidentWorkgroups / 2u ? 2.0 : 4.0;
         BuildBundleProgram(ctx, bh, P.voffs, kBundleClasses[P.cls].block, simds, P.program);

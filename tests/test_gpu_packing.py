@@ -31,8 +31,7 @@ def _run(settings, sizes, iterations=2):
         ctx.update(1 / 60, 1, 2)
         places = [ctx.placement(i) for i in ids]
         assert all(p[0] == "bundle" for p in places)
-        _run.threads = {p[1] for p in places}
-        return len({p[2] for p in places}), [ctx.read(ids[k])["pos"] for k in range(0, len(ids), 37)]
+        return len({p[2] for p in places}), {p[1] for p in places}, [ctx.read(ids[k])["pos"] for k in range(0, len(ids), 37)]
     finally:
         ctx.close()
 
@@ -42,7 +41,7 @@ def _run(settings, sizes, iterations=2):
     [5] * 513, [9] * 1023, [5, 9, 17, 31] * 200, [5] * 3000,  # at most 512, two iteration counts among them
 ], ids=lambda s: f"{len(s)}x{max(s)}")
 def test_workgroups_and_results(settings, sizes):
-    count, got = _run(settings, sizes)
+    count, _, got = _run(settings, sizes)
     print(f"{len(sizes)} bodies: {count} workgroups", flush=True)
     if len(sizes) <= AT_ONCE:
         assert count == len(sizes)
@@ -52,14 +51,16 @@ def test_workgroups_and_results(settings, sizes):
     for k, g in zip(range(0, len(sizes), 37), got):
         key = (sizes[k], k % 7 == 3)
         if key not in alone:
-            alone[key] = _run(settings, [sizes[k]], 2 + key[1])[1][0]
+            alone[key] = _run(settings, [sizes[k]], 2 + key[1])[2][0]
         assert np.array_equal(g, alone[key]), f"body {k}"
 
 
-@pytest.mark.parametrize("side, count, threads", [(17, 1, 512), (17, 256, 512), (31, 1, 1024), (31, 256, 1024), (31, 257, 512)])
-def test_threads(settings, side, count, threads):
-    """Bodies of more than 512 vertices take 1024 threads while every workgroup has a CU to itself."""
-    workgroups, got = _run(settings, [side] * count)
-    assert workgroups == count and _run.threads == {threads}
-    want = _run(settings, [side])[1][0]
-    assert all(np.array_equal(g, want) for k, g in zip(range(0, count, 37), got) if k % 7 != 3)
+@pytest.mark.parametrize("sizes, threads", [([17], {512}), ([17] * 256, {512}), ([31], {1024}), ([5] + [31] * 255, {1024}),
+                                            ([31] * 257, {512})], ids=lambda v: str(len(v)))
+def test_threads(settings, sizes, threads):
+    """Where a body has more than 512 vertices, workgroups have 1024 threads while each has a CU to itself."""
+    workgroups, used, got = _run(settings, sizes)
+    assert workgroups == len(sizes) and used == threads
+    for k, g in zip(range(0, len(sizes), 37), got):
+        want = _run(settings, [sizes[k]], 2 + (k % 7 == 3))[2][0]
+        assert np.array_equal(g, want), f"body {k}"
