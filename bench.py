@@ -12,8 +12,10 @@ resident in HBM.
 Prints one JSON line:
   metric/value/unit   constraint solves per second (sum over bodies of
                       steps x iterations x constraints, per frame)
-  roofline            algorithmic HBM bytes of the update kernels per launch /
-                      launch duration (hipEvents on the library stream)
+  roofline            algorithmic bytes of the update kernels per launch / launch
+                      duration (hipEvents on the library stream); beside them the HBM
+                      traffic that counters measured, where the record in profiles/
+                      belongs to these kernel sources
   cpu_baseline        the reference (compiled from its sources, shipped x86-64
                       flags, PhysicsSystem::Update with JobSystemThreadPool on
                       all host cores) on a bounded sample of the same workload
@@ -43,6 +45,7 @@ HBM_PEAK_GBS = 8000.0
 # collision step the plane search reads 16 B and writes 24 B).
 BYTES_EDGE, BYTES_BEND, BYTES_VOLUME, BYTES_LRA = 72, 136, 136, 48
 BYTES_VERTEX_SUBSTEP, BYTES_VERTEX_STEP = 96, 40
+ALGORITHMIC = "algorithmic bytes; those of LDS-resident bodies' positions do not move through HBM"
 
 
 def log(msg):
@@ -119,16 +122,36 @@ def cpu_baseline(scene, settings, target_seconds=15.0, max_bodies=256):
         return None
 
 
-def measured_traffic(workload):
+def kernel_sources_digest():
+    """Digest of the library's sources: which kernels a recorded counter run belongs to."""
+    import hashlib
+    csrc = os.path.join(ROOT, "joltphysics_amd", "csrc")
+    h = hashlib.sha256()
+    for name in sorted(os.listdir(csrc)):
+        if name.endswith((".h", ".hip", ".cpp")):
+            h.update(name.encode())
+            with open(os.path.join(csrc, name), "rb") as f:
+                h.update(f.read())
+    return h.hexdigest()[:16]
+
+
+def measured_traffic(workload, schedule):
     """HBM bytes per frame of the update measured with rocprofv3 FETCH_SIZE / WRITE_SIZE passes
-    (calibrated against a plain copy), as recorded in profiles/<workload>_hbm_traffic.md."""
-    path = os.path.join(os.path.dirname(os.path.abspath(__file__)), "profiles", f"{workload}_hbm_traffic.md")
+    (calibrated against a plain copy), as recorded in profiles/<workload>_hbm_traffic.md, and
+    where they come from.  None where the record was made with other kernel sources."""
+    path = os.path.join(ROOT, "profiles", f"{workload}_hbm_traffic.md")
     if not os.path.exists(path):
         return None, None
-    for line in open(path):
-        if line.startswith("traffic_bytes_per_frame:"):
-            return float(line.split(":")[1]), os.path.relpath(path, os.path.dirname(os.path.abspath(__file__)))
-    return None, None
+    record = {}
+    with open(path) as f:
+        for line in f:
+            key, _, value = line.partition(":")
+            record[key.strip()] = value.strip()
+    rel = os.path.relpath(path, ROOT)
+    if record.get("kernel_sources") != kernel_sources_digest():
+        return None, f"{rel} was measured with other kernel sources"
+    value = record.get(f"traffic_bytes_per_frame_{schedule}")
+    return (float(value), rel) if value else (None, None)
 
 
 DIGESTS = {"exact": "batched2048_sample_digests.json", "coloured": "batched2048_coloured_sample_digests.json"}
@@ -357,18 +380,25 @@ def main():
         # the coloured schedule on the same workload: fewer, wider level passes
         t_wall, t_launch, t_kernel_ms, t_parity = timed_run(scene, settings, "coloured", args.warmup, args.steps)
         t_achieved = algorithmic_bytes_per_frame(scene, settings) * args.steps / (t_kernel_ms / 1000.0) / 1e9
+        t_traffic, t_src = measured_traffic(scene.name, "coloured")
         throughput = {"schedule": "coloured", "value": solves * args.steps / t_wall, "unit": "constraint-solves/s",
                       "ms_per_step": 1000.0 * t_wall / args.steps, "launch_ms": round(t_kernel_ms / max(t_launch, 1), 3),
                       "roofline": {"bound": "hbm", "achieved": round(t_achieved, 2), "peak": HBM_PEAK_GBS, "unit": "GB/s",
-                                   "frac": round(t_achieved / HBM_PEAK_GBS, 4)},
+                                   "frac": round(t_achieved / HBM_PEAK_GBS, 4),
+                                   "traffic": None if t_traffic is None else t_traffic * args.steps,
+                                   "traffic_gbs": None if t_traffic is None else
+                                   round(t_traffic * args.steps / (t_kernel_ms / 1000.0) / 1e9, 2),
+                                   "traffic_source": t_src, "achieved_counts": ALGORITHMIC},
                       "parity": t_parity}
     bytes_frame = algorithmic_bytes_per_frame(scene, settings)
     achieved = bytes_frame * args.steps / (kernel_ms / 1000.0) / 1e9
-    traffic, traffic_src = measured_traffic(scene.name)
+    traffic, traffic_src = measured_traffic(scene.name, args.schedule)
     roofline = {"bound": "hbm", "achieved": round(achieved, 2), "peak": HBM_PEAK_GBS, "unit": "GB/s",
                 "frac": round(achieved / HBM_PEAK_GBS, 4),
                 "traffic": None if traffic is None else traffic * args.steps,
+                "traffic_gbs": None if traffic is None else round(traffic * args.steps / (kernel_ms / 1000.0) / 1e9, 2),
                 "traffic_source": traffic_src,
+                "achieved_counts": ALGORITHMIC,
                 "kernel": "one xpbd_update: bundle_kernel launches (one per launch class) + update_kernel (streamed "
                           "bodies), concurrent on one stream per hardware queue, timed fork to join",
                 "algorithmic_bytes_per_launch": bytes_frame * args.steps,

@@ -57,8 +57,8 @@ __host__ __device__ inline TeamLds team_lds_layout(uint32_t window_capacity, uin
 // count these among the pending memory operations: after a wait that leaves none pending it
 // removes the wait that belongs to the fence, and the members would be counted in while their
 // stores are still on their way out of the XCD's L2 (a long way where other launches have filled it
-// with dirty lines).  Both waits together: 17.9 -> 18.3 ms on a 40-cell block with 56 barriers in each of
-// 40 sub-steps, 0.2 us a barrier.
+// with dirty lines).  Both waits together cost 0.2 us a barrier for 16 members (40-cell block, 56 barriers
+// in each of 40 sub-steps: 17.9 -> 18.3 ms), 0.5 us for 56 (64-cell block, 57 in 80: 50.9 -> 53.3 ms).
 __device__ __forceinline__ void wait_cache_operation() { asm volatile("s_waitcnt vmcnt(0)" ::: "memory"); }
 
 // Team barrier.  `target` = team size x number of this barrier in the launch.
