@@ -1,7 +1,8 @@
 """Task programs on the GPU: both forms of every projection (one lane and four lanes per
 constraint), ragged and tiny levels, levels of one wavefront in a row, one or many bodies per
-workgroup, and values at the ends of the float range, where a shared division falls back to the
-plain one.  Bit-exact against the restatement (FP32)."""
+workgroup, and values at the ends of the float range (of bodies whose bends all run on four lanes; wide
+levels and the fall-back of their shared divisions: test_gpu_wide_tasks.py).  Bit-exact against the
+restatement (FP32)."""
 import numpy as np
 import pytest
 
