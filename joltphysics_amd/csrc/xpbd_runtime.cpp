@@ -10,6 +10,7 @@
 #include <cstring>
 #include <memory>
 #include <string>
+#include <unordered_map>
 #include <vector>
 #include <limits>
 
@@ -3362,8 +3363,10 @@ int xpbd_rollout_create(xpbd_context *ctx, const xpbd_rollout_desc *d, xpbd_roll
     std::vector<float4> x0;
     std::vector<RolloutBodyDev> bodies(d->num_bodies);
     TaskProgram tp;
-    struct TaskFirst { size_t recs, desc, heads; };
+    struct TaskFirst { size_t recs, desc, heads, host_recs; };     // device offsets; records: where tp holds them
+    size_t num_task_recs = 0;
     std::vector<TaskFirst> first(d->num_bodies);
+    std::unordered_map<xpbd_settings *, uint32_t> first_of;     // the first body of each settings
     size_t tape = 0;            // float4 of one sub-step's tape
     for (uint32_t b = 0; b < d->num_bodies; ++b)
         if (d->settings[b])
@@ -3387,37 +3390,46 @@ int xpbd_rollout_create(xpbd_context *ctx, const xpbd_rollout_desc *d, xpbd_roll
         B.num_edges = ne;
         B.voff = r->total_nv;
         B.eoff = r->total_ne;
+        // bodies of the same settings share the level program of the double pass, which is only read, and
+        // the task program of the float passes but for its records, which hold each body's compliances
+        // (64 cloths of 64 x 64: 1.2 ms for the rollout, 17 with programs and uploads of their own)
+        const uint32_t same = first_of.emplace(s, b).first->second;
         const size_t rbase = recs.size();
         B.nlev = (uint32_t)s->host_level_begin.size() - 1;
         B.num_records = (uint32_t)s->host_recs.size();
-        B.lvl = reinterpret_cast<const uint32_t *>((uintptr_t)lvl.size());     // index until uploaded
         B.num_faces = nf;
         B.pressure = d->pressure;
         B.faces = s->faces.p;           // the settings' device arrays (the rollout holds a reference)
         B.vf_begin = s->vf_begin.p;
         B.vf_list = s->vf_list.p;
-        for (uint32_t L : s->host_level_begin)
-            lvl.push_back(L);                       // relative to the body's first record
         B.edges_only = s->num_volumes + s->num_bends + s->num_lras == 0 ? 1u : 0u;
-        for (size_t k = 0; k < s->host_recs.size(); ++k)
+        if (same == b)
         {
-            uint4 q = s->host_recs[k];
-            if (q.x != kNopRecordHost && ((q.x >> 14) & 3u) != kTypeVolume && ((q.x >> 14) & 3u) != kTypeBend)
+            B.lvl = reinterpret_cast<const uint32_t *>((uintptr_t)lvl.size());     // index until uploaded
+            for (uint32_t L : s->host_level_begin)
+                lvl.push_back(L);                       // relative to the body's first record
+            for (size_t k = 0; k < s->host_recs.size(); ++k)
             {
-                // edges: their index in the body (for the compliance parameters) and a compliance
-                // written by each float forward pass; LRAs: their index.  Volume and bend records
-                // keep their vertices 2-3 and parameters.
-                q.y = s->host_rec_index[k];
-                q.w = 0u;
+                uint4 q = s->host_recs[k];
+                if (q.x != kNopRecordHost && ((q.x >> 14) & 3u) != kTypeVolume && ((q.x >> 14) & 3u) != kTypeBend)
+                {
+                    // edges: their index in the body (for the compliance parameters) and room for the
+                    // compliance that the float forward pass writes into its copy; LRAs: their index.
+                    // Volume and bend records keep their vertices 2-3 and parameters.
+                    q.y = s->host_rec_index[k];
+                    q.w = 0u;
+                }
+                recs.push_back(q);
             }
-            recs.push_back(q);
+            B.recs = reinterpret_cast<const uint4 *>((uintptr_t)rbase);
         }
-        B.recs = reinterpret_cast<const uint4 *>((uintptr_t)rbase);
-        // task program of the float passes; bodies of the same settings share it but for the
-        // records, which hold each body's compliances
+        else
+        {
+            B.lvl = bodies[same].lvl;
+            B.recs = bodies[same].recs;
+        }
         {
             TaskProgram own;
-            const uint32_t same = b > 0 && d->settings[b - 1] == s ? b - 1 : b;
             if (same == b)
             {
                 TaskBuilder builder(waves, 4.0);
@@ -3429,7 +3441,7 @@ int xpbd_rollout_create(xpbd_context *ctx, const xpbd_rollout_desc *d, xpbd_roll
                     builder.Level(bucket, true);
                 }
                 builder.Finish(own);
-                first[b] = { tp.recs.size(), tp.desc.size(), tp.heads.size() };
+                first[b] = { num_task_recs, tp.desc.size(), tp.heads.size(), tp.recs.size() };
                 B.num_task_records = (uint32_t)own.recs.size() - 1u;
                 tp.recs.insert(tp.recs.end(), own.recs.begin(), own.recs.end());
                 tp.desc.insert(tp.desc.end(), own.desc.begin(), own.desc.end());
@@ -3437,12 +3449,10 @@ int xpbd_rollout_create(xpbd_context *ctx, const xpbd_rollout_desc *d, xpbd_roll
             }
             else
             {
-                first[b] = { tp.recs.size(), first[same].desc, first[same].heads };
+                first[b] = { num_task_recs, first[same].desc, first[same].heads, 0 };
                 B.num_task_records = bodies[same].num_task_records;
-                const size_t n = B.num_task_records + 1u;
-                tp.recs.resize(first[b].recs + n);
-                std::copy_n(tp.recs.begin() + first[same].recs, n, tp.recs.begin() + first[b].recs);
             }
+            num_task_recs += B.num_task_records + 1u;
             // edges and LRAs keep one float4 per record and sub-step, volumes and bends three
             B.tape_stride = s->num_volumes + s->num_bends > 0 ? 3u : 1u;
             B.tape_offset = tape;
@@ -3459,7 +3469,18 @@ int xpbd_rollout_create(xpbd_context *ctx, const xpbd_rollout_desc *d, xpbd_roll
     HIP_TRY(r->recs.upload(recs));
     HIP_TRY(r->lvl.upload(lvl));
     HIP_TRY(r->x0.upload(x0));
-    HIP_TRY(r->task_recs.upload(tp.recs));
+    // the records of one body per settings go up, the others' are copied on the device
+    HIP_TRY(r->task_recs.alloc(num_task_recs));
+    for (uint32_t b = 0; b < d->num_bodies; ++b)
+    {
+        const uint32_t same = first_of[d->settings[b]];
+        const size_t bytes = sizeof(uint4) * (bodies[b].num_task_records + 1u);
+        if (same == b)
+            HIP_TRY(hipMemcpy(r->task_recs.p + first[b].recs, tp.recs.data() + first[b].host_recs, bytes, hipMemcpyHostToDevice));
+        else
+            HIP_TRY(hipMemcpyAsync(r->task_recs.p + first[b].recs, r->task_recs.p + first[same].recs, bytes, hipMemcpyDeviceToDevice, nullptr));
+    }
+    HIP_TRY(hipStreamSynchronize(nullptr));
     HIP_TRY(r->task_desc.upload(tp.desc));
     HIP_TRY(r->task_heads.upload(tp.heads));
     for (uint32_t b = 0; b < d->num_bodies; ++b)
