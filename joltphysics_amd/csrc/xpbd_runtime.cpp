@@ -10,9 +10,11 @@
 #include <cstring>
 #include <memory>
 #include <string>
+#include <type_traits>
 #include <unordered_map>
 #include <vector>
 #include <limits>
+#include <map>
 
 #include "../../include/jolt_xpbd.h"
 #include "jolt_math.h"
@@ -201,16 +203,10 @@ struct BundleHost
     uint32_t nv = 0;
     bool uniform = false;
     float inv_mass = 0.0f;
-    DevBuf<uint4> recs, heads;
-    DevBuf<uint32_t> desc;
-    DevBuf<BundleBodyDev> table;
-    DevBuf<float4> x, v, prev, plane, report, face_normals;
-    DevBuf<uint2> faces;
-    DevBuf<uint32_t> vf_begin, vf_list;
-    DevBuf<float> face_terms;
-    DevBuf<int32_t> idx, contact;
-    DevBuf<unsigned char> leaves_full, leaves;
-    BundleDev dev{};
+    // everything the bundle has on the device, in one allocation: what is uploaded, then vertex state,
+    // leaves and face scratch (an allocation and an upload for each took 60 us of a layout's time)
+    DevBuf<unsigned char> storage;
+    BundleDev dev{};            // pointers into it
 };
 
 struct xpbd_context
@@ -1626,13 +1622,14 @@ int BuildLayout(xpbd_context *ctx)
     struct Plan
     {
         std::vector<uint32_t> voffs;
-        TaskProgram program;
+        std::shared_ptr<TaskProgram> program;
         uint32_t iterations, foff;
         bool has_pressure, has_sleepers;
         int cls;
         double us;              // estimated µs per collision step
     };
     std::vector<Plan> plans(bundles.size());
+    std::map<std::pair<const xpbd_settings *, int>, std::shared_ptr<TaskProgram>> alone;
     for (size_t k = 0; k < bundles.size(); ++k)
     {
         BundleHost &bh = *bundles[k];
@@ -1664,8 +1661,21 @@ int BuildLayout(xpbd_context *ctx)
         P.cls = lds <= kBundleClasses[0].lds && !wide ? 0 : 1;
         // workgroups that share a CU share its four SIMDs
         const double simds = P.cls == 0 && bundles.size() > kResidentWorkgroups / 2u ? 2.0 : 4.0;
-        BuildBundleProgram(ctx, bh, P.voffs, kBundleClasses[P.cls].block, simds, P.program);
-        P.us = 1e-3 * P.program.ns * P.iterations;
+        // bodies of the same settings that are alone in their workgroups have the same program (but for
+        // skinned ones, whose records hold the number of their first skin entry)
+        const Body &first = *ctx->bodies[bh.bodies[0]];
+        const auto key = std::make_pair((const xpbd_settings *)first.settings, P.cls);
+        const bool shared = nb == 1 && first.settings->skinned.empty();
+        if (shared && alone.count(key))
+            P.program = alone[key];
+        else
+        {
+            P.program = std::make_shared<TaskProgram>();
+            BuildBundleProgram(ctx, bh, P.voffs, kBundleClasses[P.cls].block, simds, *P.program);
+            if (shared)
+                alone[key] = P.program;
+        }
+        P.us = 1e-3 * P.program->ns * P.iterations;
     }
 
     HIP_TRY(ctx->d_elapsed.alloc(std::max<size_t>(1, bundles.size())));
@@ -1698,32 +1708,11 @@ int BuildLayout(xpbd_context *ctx)
                 foff += b.settings->num_faces;
         }
         const uint32_t voff = bh.nv;
-        HIP_TRY(bh.recs.upload(P.program.recs));
-        HIP_TRY(bh.desc.upload(P.program.desc));
-        HIP_TRY(bh.heads.upload(P.program.heads));
-        HIP_TRY(bh.table.upload(table));
-        // bundle-contiguous vertex state, gathered from wherever each body's state lives now
-        HIP_TRY(bh.x.alloc(voff)); HIP_TRY(bh.v.alloc(voff)); HIP_TRY(bh.prev.alloc(voff)); HIP_TRY(bh.plane.alloc(voff));
-        HIP_TRY(bh.report.alloc(voff));
-        HIP_TRY(bh.idx.alloc(voff)); HIP_TRY(bh.contact.alloc(voff));
-        for (uint32_t j = 0; j < nb; ++j)
-        {
-            Body &b = *ctx->bodies[bh.bodies[j]];
-            const size_t o = P.voffs[j], n = b.nv;
-            HIP_TRY(hipMemcpy(bh.x.p + o, b.dev.x, n * sizeof(float4), hipMemcpyDeviceToDevice));
-            HIP_TRY(hipMemcpy(bh.v.p + o, b.dev.v, n * sizeof(float4), hipMemcpyDeviceToDevice));
-            HIP_TRY(hipMemcpy(bh.prev.p + o, b.dev.prev, n * sizeof(float4), hipMemcpyDeviceToDevice));
-            HIP_TRY(hipMemcpy(bh.plane.p + o, b.dev.plane, n * sizeof(float4), hipMemcpyDeviceToDevice));
-            HIP_TRY(hipMemcpy(bh.report.p + o, b.dev.report, n * sizeof(float4), hipMemcpyDeviceToDevice));
-            HIP_TRY(hipMemcpy(bh.idx.p + o, b.dev.idx, n * sizeof(int32_t), hipMemcpyDeviceToDevice));
-            HIP_TRY(hipMemcpy(bh.contact.p + o, b.dev.contact, n * sizeof(int32_t), hipMemcpyDeviceToDevice));
-        }
-        HIP_TRY(bh.leaves_full.alloc((size_t)std::max(1u, nb * nc) * bundle_leaf_bytes()));
-        HIP_TRY(bh.leaves.alloc((size_t)std::max(1u, nb * nc) * bundle_leaf_bytes()));
+        std::vector<uint2> faces;
+        std::vector<uint32_t> vf_begin, vf_list;
         if (P.has_pressure)
         {
-            std::vector<uint2> faces;
-            std::vector<uint32_t> vf_begin(1, 0u), vf_list;
+            vf_begin.push_back(0u);
             faces.reserve(P.foff);
             for (uint32_t j = 0; j < nb; ++j)
             {
@@ -1743,19 +1732,52 @@ int BuildLayout(xpbd_context *ctx)
                     vf_begin.push_back((uint32_t)vf_list.size());
                 }
             }
-            HIP_TRY(bh.faces.upload(faces));
-            HIP_TRY(bh.vf_begin.upload(vf_begin));
-            HIP_TRY(bh.vf_list.upload(vf_list));
-            HIP_TRY(bh.face_normals.alloc(faces.size()));
-            HIP_TRY(bh.face_terms.alloc(faces.size()));
         }
         BundleDev &d = bh.dev;
-        d.recs = bh.recs.p; d.desc = bh.desc.p; d.heads = bh.heads.p;
-        d.bodies = bh.table.p; d.num_bodies = nb; d.nv = voff;
-        d.x = bh.x.p; d.v = bh.v.p; d.prev = bh.prev.p; d.plane = bh.plane.p; d.idx = bh.idx.p; d.contact = bh.contact.p;
-        d.report = bh.report.p;
-        d.leaves_full = bh.leaves_full.p; d.leaves = bh.leaves.p; d.faces = bh.faces.p; d.num_faces = P.has_pressure ? P.foff : 0u; d.vf_begin = bh.vf_begin.p; d.vf_list = bh.vf_list.p;
-        d.face_normals = bh.face_normals.p; d.face_terms = bh.face_terms.p;
+        size_t size = 0;
+        auto reserve = [&](size_t bytes) {
+            const size_t o = size;
+            size += (bytes + 255u) / 256u * 256u;
+            return o;
+        };
+        std::vector<unsigned char> image;
+        auto place = [&](const void *data, size_t bytes) {
+            const size_t o = reserve(bytes);
+            image.resize(size);
+            if (bytes)
+                memcpy(image.data() + o, data, bytes);
+            return o;
+        };
+        auto place_all = [&](const auto &v) { return place(v.data(), v.size() * sizeof(v[0])); };
+        const size_t recs = place_all(P.program->recs), desc = place_all(P.program->desc), heads = place_all(P.program->heads);
+        const size_t bodies = place_all(table), face_list = place_all(faces), vfb = place_all(vf_begin), vfl = place_all(vf_list);
+        const size_t vec = sizeof(float4) * voff, leaf = (size_t)std::max(1u, nb * nc) * bundle_leaf_bytes();
+        const size_t x = reserve(vec), v = reserve(vec), prev = reserve(vec), plane = reserve(vec), report = reserve(vec);
+        const size_t idx = reserve(sizeof(int32_t) * voff), contact = reserve(sizeof(int32_t) * voff);
+        const size_t leaves_full = reserve(leaf), leaves = reserve(leaf);
+        const size_t normals = reserve(sizeof(float4) * faces.size()), terms = reserve(sizeof(float) * faces.size());
+        HIP_TRY(bh.storage.alloc(size));
+        HIP_TRY(hipMemcpy(bh.storage.p, image.data(), image.size(), hipMemcpyHostToDevice));
+        auto at = [&](size_t o, auto *&pointer) { pointer = reinterpret_cast<std::remove_reference_t<decltype(pointer)>>(bh.storage.p + o); };
+        at(recs, d.recs); at(desc, d.desc); at(heads, d.heads); at(bodies, d.bodies);
+        at(face_list, d.faces); at(vfb, d.vf_begin); at(vfl, d.vf_list);
+        at(x, d.x); at(v, d.v); at(prev, d.prev); at(plane, d.plane); at(report, d.report); at(idx, d.idx); at(contact, d.contact);
+        d.leaves_full = bh.storage.p + leaves_full; d.leaves = bh.storage.p + leaves;
+        at(normals, d.face_normals); at(terms, d.face_terms);
+        d.num_bodies = nb; d.nv = voff; d.num_faces = P.has_pressure ? P.foff : 0u;
+        // bundle-contiguous vertex state, gathered from wherever each body's state lives now
+        for (uint32_t j = 0; j < nb; ++j)
+        {
+            Body &b = *ctx->bodies[bh.bodies[j]];
+            const size_t o = P.voffs[j], n = b.nv;
+            HIP_TRY(hipMemcpy(d.x + o, b.dev.x, n * sizeof(float4), hipMemcpyDeviceToDevice));
+            HIP_TRY(hipMemcpy(d.v + o, b.dev.v, n * sizeof(float4), hipMemcpyDeviceToDevice));
+            HIP_TRY(hipMemcpy(d.prev + o, b.dev.prev, n * sizeof(float4), hipMemcpyDeviceToDevice));
+            HIP_TRY(hipMemcpy(d.plane + o, b.dev.plane, n * sizeof(float4), hipMemcpyDeviceToDevice));
+            HIP_TRY(hipMemcpy(d.report + o, b.dev.report, n * sizeof(float4), hipMemcpyDeviceToDevice));
+            HIP_TRY(hipMemcpy(d.idx + o, b.dev.idx, n * sizeof(int32_t), hipMemcpyDeviceToDevice));
+            HIP_TRY(hipMemcpy(d.contact + o, b.dev.contact, n * sizeof(int32_t), hipMemcpyDeviceToDevice));
+        }
         d.has_pressure = P.has_pressure ? 1u : 0u;
         d.has_sleepers = P.has_sleepers ? 1u : 0u;
         d.iterations = P.iterations;
@@ -1782,8 +1804,8 @@ int BuildLayout(xpbd_context *ctx)
             Body &b = *ctx->bodies[bp->bodies[j]];
             uint32_t o = 0;
             for (uint32_t k = 0; k < j; ++k) o += ctx->bodies[bp->bodies[k]]->nv;
-            b.dev.x = bp->x.p + o; b.dev.v = bp->v.p + o; b.dev.prev = bp->prev.p + o; b.dev.plane = bp->plane.p + o;
-            b.dev.idx = bp->idx.p + o; b.dev.contact = bp->contact.p + o; b.dev.report = bp->report.p + o;
+            b.dev.x = bp->dev.x + o; b.dev.v = bp->dev.v + o; b.dev.prev = bp->dev.prev + o; b.dev.plane = bp->dev.plane + o;
+            b.dev.idx = bp->dev.idx + o; b.dev.contact = bp->dev.contact + o; b.dev.report = bp->dev.report + o;
             if (b.owns_storage)
             {
                 (void)b.x.alloc(0); (void)b.v.alloc(0); (void)b.prev.alloc(0); (void)b.plane.alloc(0); (void)b.idx.alloc(0); (void)b.contact.alloc(0);

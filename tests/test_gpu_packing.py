@@ -64,3 +64,23 @@ def test_threads(settings, sizes, threads):
     for k, g in zip(range(0, len(sizes), 37), got):
         want = _run(settings, [sizes[k]], 2 + (k % 7 == 3))[2][0]
         assert np.array_equal(g, want), f"body {k}"
+
+
+def test_layout_costs_less_than_the_bodies(settings):
+    """Laying out many small bodies, a workgroup each, takes less than creating them."""
+    import time
+    create = layout = 1e9
+    for _ in range(4):
+        ctx = Context(0)
+        st = ctx.create_settings(settings[17])
+        t0 = time.perf_counter()
+        for k in range(400):
+            ctx.create_body(st, (2.0 * k, 0.0, 1.0), (0.0, 0.0, 0.0, 1.0), BodyParams(allow_sleeping=False))
+        t1 = time.perf_counter()
+        ctx.update(1 / 60, 1, 1)
+        ctx.synchronize()
+        create, layout = min(create, t1 - t0), min(layout, time.perf_counter() - t1)
+        ctx.close()
+    print(f"400 bodies: created in {1e3 * create:.1f} ms, first update {1e3 * layout:.1f} ms", flush=True)
+    # 25 against 37 ms; 55 with eleven allocations, four uploads and a program built for every workgroup
+    assert layout < create
