@@ -1509,10 +1509,16 @@ int BuildTeams(xpbd_context *ctx)
 constexpr size_t kReadHeader = (sizeof(ReadHeader) + 255) / 256 * 256;
 constexpr size_t kReadVertex = 15 * 4;
 
+// Pinned memory for reads of `bytes`; where there is too little, for a whole read of the context's
+// largest body, so that reads of ever larger bodies do not pin memory each.
 int ReserveRead(xpbd_context *ctx, size_t bytes)
 {
     if (ctx->h_read_n >= bytes)
         return XPBD_OK;
+    size_t largest = 0;
+    for (const auto &b : ctx->bodies)
+        largest = std::max<size_t>(largest, b->nv);
+    bytes = std::max(bytes, kReadHeader + kReadVertex * largest);
     if (ctx->h_read)
         HIP_TRY(hipHostFree(ctx->h_read));
     ctx->h_read = nullptr;
@@ -1524,7 +1530,7 @@ int ReserveRead(xpbd_context *ctx, size_t bytes)
 
 int BuildLayout(xpbd_context *ctx)
 {
-    // once for the largest body here, so that no read has to pin memory
+    // here, so that no read has to pin memory
     size_t largest = 0;
     for (const auto &b : ctx->bodies)
         largest = std::max<size_t>(largest, b->nv);
@@ -2829,7 +2835,7 @@ int xpbd_body_read(xpbd_context *ctx, int32_t body, float *pos, float *prev, flo
     Body &b = *ctx->bodies[body];
     const size_t nv = b.nv;
     const size_t words = nv * ((pos ? 3 : 0) + (prev ? 3 : 0) + (vel ? 3 : 0) + (plane ? 4 : 0) + (shape_idx ? 1 : 0) + (contact ? 1 : 0));
-    // before the first update of a layout there may be no buffer, or one for smaller bodies
+    // before the bodies' first update there may be no buffer, or one for smaller bodies
     if (int rc = ReserveRead(ctx, kReadHeader + 4 * words))
         return rc;
     // the body's row of the device states; without one (no update since it was created) the host's is current
