@@ -1228,7 +1228,9 @@ int BuildSchedule(const xpbd_settings_desc &d, xpbd_settings &s, int32_t schedul
             || (e = s.d_skinned_normals.upload(s.skinned_normals)) != hipSuccess)
             return Fail(XPBD_E_DEVICE, std::string("settings upload: ") + hipGetErrorString(e));
     }
-    if ((e = s.recs.upload(pb.recs)) != hipSuccess || (e = s.lvl.upload(pb.lvl)) != hipSuccess
+    // the windows of streamed bodies without rods run as task programs, every other body's as levels
+    const bool window_tasks = !resident && d.num_rod_stretch_shear == 0;
+    if ((!window_tasks && ((e = s.recs.upload(pb.recs)) != hipSuccess || (e = s.lvl.upload(pb.lvl)) != hipSuccess))
         || (e = s.windows.upload(pb.windows)) != hipSuccess || (e = s.vlist.upload(pb.vlist)) != hipSuccess
         || (e = s.faces.upload(f3)) != hipSuccess || (e = s.vf_begin.upload(vf_begin)) != hipSuccess
         || (e = s.vf_list.upload(vf_list)) != hipSuccess)
@@ -1260,10 +1262,10 @@ int BuildSchedule(const xpbd_settings_desc &d, xpbd_settings &s, int32_t schedul
         s.rods.assign(rods, rods + d.num_rod_stretch_shear);
     }
 
-    // task programs of the gathered windows (bodies with rods run the level programs)
-    if (!resident && d.num_rod_stretch_shear == 0)
+    if (window_tasks)
     {
         TaskProgram tp;
+        tp.recs.reserve(pb.recs.size() + 1u);
         std::vector<uint4> bucket[4];
         for (const WindowDev &w : pb.windows)
         {
